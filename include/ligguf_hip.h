@@ -246,11 +246,11 @@ int lg_prefill(lg_ctx* ctx, const int* toks, int n, int pos0, float* logits_host
  * int8 MFMA GEMMs, the tokens' integer sub-block sums and quantizers those
  * of the step; the logits then match n sequential steps to fp32 rounding (an
  * int8 rounding of an activation may differ in rare tokens).  Takes every
- * layer type -- Q2_K..Q6_K, Q8_0, Q1_0, Q1_G on int8 MFMA, F32/F16 on fp32
- * MFMA, in any mix (a Q4_K_M-style model with Q6_K matrices among its Q4_K
- * ones included) -- and needs head_dim 48, 64 or 128 with 1, 2, 4 or 8 query
- * heads per KV head.  STEPS: one
- * decode step per token, bit-equal to n lg_decode_step calls.  AUTO (the
+ * layer type -- Q2_K..Q6_K, Q8_0, Q1_0, Q1_G on int8 MFMA, F16 on fp16
+ * MFMA (each fp32 activation as two fp16 parts), F32 on fp32 MFMA, in any
+ * mix (a Q4_K_M-style model with Q6_K matrices among its Q4_K ones included)
+ * -- and needs head_dim 48, 64 or 128 with 1, 2, 4 or 8 query heads per KV
+ * head.  STEPS: one decode step per token, bit-equal to n lg_decode_step calls.  AUTO (the
  * default): BATCHED when the model allows it and n >= 2, else STEPS.
  * lg_prefill_path reports what a prompt of 2+ tokens takes (-1 without a
  * model). */
@@ -310,7 +310,8 @@ int lg_matvec(int type, const void* w, uint32_t rsz, int n, int d, const void* x
  * out[t*d + r] = row r of w . Q(x[t*n ..]) for t < T, r < d, each fp32 row
  * of x quantized as quantize_q8_K (K-quant weights, n % 256 == 0) or
  * quantize_q8_0 (Q8_0, Q1_0, Q1_G weights; n % 32 == 0, n % 256 for Q1_G)
- * does, or taken as fp32 (F32/F16 weights, n % 32 == 0, on fp32 MFMA).  The
+ * does, or taken as fp32 (F32 weights on fp32 MFMA, F16 weights on fp16 MFMA
+ * with each value in two fp16 parts; n % 32 == 0).  The
  * integer block sums are those of lg_matvec (the dot products of
  * fast/lil_math.cpp:397-739); only the fp32 accumulation order differs.  Allocates and frees a workspace of
  * about 1.3*T*n bytes and synchronizes `stream` (tests and benches).  No

@@ -38,6 +38,7 @@
 #include <vector>
 
 #include "lg_common.h"
+#include "lg_fgemm.h"
 #include "lg_prefill.h"
 #include "lg_quant.h"
 
@@ -202,25 +203,6 @@ __global__ __launch_bounds__(256) void k_bert_quant(const float* __restrict__ x,
 /* ------------------------------------------------------------------ */
 /* token-batched GEMM: out[t][r] = W[r] . act[t] (+ epilogue)           */
 /* ------------------------------------------------------------------ */
-enum { EP_BIAS = 0, EP_BIAS_RES = 1, EP_BIAS_GELU = 2, EP_STORE = 3, EP_ADD = 4 };   /* STORE/ADD: no bias; ADD: out += */
-
-struct BGemm {
-    const uint8_t* w;          /* F32/F16: [R][K]; BF_I8: int8 [R][K] */
-    const float* wd;           /* BF_I8: [K/32][R] */
-    int R, K;
-    const float* x;            /* fp32 activations [T][ldx] (F32/F16) */
-    int ldx;
-    const int8_t* q;           /* Q8_0 activations [T][K] (BF_I8) */
-    const float* qd;           /* [K/32][ldd] */
-    int ldd;
-    int T;
-    const float* bias;         /* [R] */
-    const float* res;          /* [T][ldr] residual (EP_BIAS_RES) */
-    int ldr;
-    float* out;                /* [T][ldo] */
-    int ldo;
-};
-
 /* One wave per (16 TM)-token x (16 TN)-row tile (TM x TN MFMA tiles of
  * 16 x 16; the launcher picks the largest tile that still gives the grid
  * enough waves).  MFMA operand A holds tokens (M), B weight rows (N); the
@@ -1167,25 +1149,19 @@ static int gemm_ep(const BMat& W, const float* x, int ldx, const lg_bert* b, int
     return lg_check_launch("bert gemm");
 }
 
-/* The same GEMM for the batched prefill's F32/F16 layer matrices
+/* The same GEMM for the batched prefill's F32 layer matrices
  * (lg_prefill.h): out[t][r] (+)= W[r] . x[t], fp32 activations. */
-int lg_fgemm_tokens(int wtype, const uint8_t* W, int rows, int cols, const float* x, int ldx, int T, float* out, int ldo,
+int lg_fgemm_tokens(const uint8_t* W, int rows, int cols, const float* x, int ldx, int T, float* out, int ldo,
                     int accumulate, hipStream_t s)
 {
-    if ((wtype != LG_F32 && wtype != LG_F16) || !W || !x || !out || rows <= 0 || cols <= 0 || cols % 32 || T <= 0 ||
-        ldx < cols || ldx % 4 || ldo < rows) {
-        lg_set_error("fp gemm: bad arguments (type %d, rows %d, cols %d, T %d)", wtype, rows, cols, T);
+    if (!W || !x || !out || rows <= 0 || cols <= 0 || cols % 32 || T <= 0 || ldx < cols || ldx % 4 || ldo < rows) {
+        lg_set_error("fp gemm: bad arguments (rows %d, cols %d, T %d)", rows, cols, T);
         return LG_ERR_ARG;
     }
     BGemm a = {};
     a.w = W; a.R = rows; a.K = cols; a.x = x; a.ldx = ldx; a.T = T; a.out = out; a.ldo = ldo;
-    if (wtype == LG_F32) {
-        if (accumulate) gemm_tiles<LG_F32, EP_ADD>(a, s);
-        else gemm_tiles<LG_F32, EP_STORE>(a, s);
-    } else {
-        if (accumulate) gemm_tiles<LG_F16, EP_ADD>(a, s);
-        else gemm_tiles<LG_F16, EP_STORE>(a, s);
-    }
+    if (accumulate) gemm_tiles<LG_F32, EP_ADD>(a, s);
+    else gemm_tiles<LG_F32, EP_STORE>(a, s);
     return lg_check_launch("fp gemm");
 }
 

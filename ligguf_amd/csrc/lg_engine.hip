@@ -917,7 +917,7 @@ extern "C" int lg_decode_path(const lg_ctx* ctx)
 #define LG_PF_TMAX 512   /* tokens per layer pass */
 
 /* the batched prefill serves models whose layer matrices all have a batched
- * GEMM (the K-quants, Q8_0, Q1_0, Q1_G on int8 MFMA, F32/F16 on fp32 MFMA;
+ * GEMM (the K-quants, Q8_0, Q1_0, Q1_G on int8, F16 on fp16, F32 on fp32 MFMA;
  * any mix, Q|K|V and up|gate stacked or not) and whose attention shape the
  * prefill attention kernel takes */
 static PfMat pf_mat(const dweight& w) { return PfMat{w.data, w.rsz, w.type, w.rows}; }
@@ -932,7 +932,7 @@ static void setup_prefill(lg_ctx* ctx, const lg_model_desc* m)
         const int at = lg_prefill_act_type(w.type);
         /* the Q1_G GEMM steps 256 values */
         if (at < 0 || (w.type == LG_Q1_G && w.cols % 256)) ok = false;
-        fam |= at == LG_Q8_K ? 1 : at == LG_Q8_0 ? 2 : 4;
+        fam |= at == LG_Q8_K ? 1 : at == LG_Q8_0 ? 2 : at == LG_F32 ? 4 : 8;
     };
     for (int l = 0; ok && l < m->n_layers; l++) {
         const dlayer& D = ctx->layers[l];
@@ -1012,9 +1012,14 @@ static int prefill_buffers(lg_ctx* c)
         if ((rc = dalloc(c, (void**)&B.qk.bs, (size_t)tmax * (wide / 256) * 16 * 2))) return rc;
         B.qk.tld = tmax;
     }
-    if (c->pf_fam & 4) {   /* F32/F16 weights: the fp32 activations */
+    if (c->pf_fam & 4) {   /* F32 weights: the fp32 activations */
         if ((rc = dalloc(c, (void**)&B.qf.f, (size_t)tmax * wide * 4))) return rc;
         B.qf.tld = tmax;
+    }
+    if (c->pf_fam & 8) {   /* F16 weights: the fp32 activations as two fp16 parts, a scale per token */
+        if ((rc = dalloc(c, (void**)&B.qh.hs.h, lg_hsplit_bytes(tmax, (int)wide)))) return rc;
+        if ((rc = dalloc(c, (void**)&B.qh.hs.inv, (size_t)tmax * 4))) return rc;
+        B.qh.tld = tmax;
     }
     if (c->pf_fam & 2) {   /* Q8_0: quants, a scale and a sum per 32 values */
         if ((rc = dalloc(c, (void**)&B.q0.qs, (size_t)tmax * wide))) return rc;
@@ -1582,14 +1587,18 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
         return LG_ERR_ARG;
     }
     if (at == LG_F32) {   /* fp32 activations as given */
-        if (rsz != (uint32_t)n * (type == LG_F32 ? 4u : 2u)) {
+        if (rsz != (uint32_t)n * 4u) {
             lg_set_error("matmul_tokens: row bytes %u for %d values", rsz, n);
             return LG_ERR_ARG;
         }
-        int rc = lg_fgemm_tokens(type, (const uint8_t*)w, d, n, x, n, T, out, d, 0, (hipStream_t)stream);
+        int rc = lg_fgemm_tokens((const uint8_t*)w, d, n, x, n, T, out, d, 0, (hipStream_t)stream);
         const hipError_t e2 = hipStreamSynchronize((hipStream_t)stream);
         if (!rc && e2 != hipSuccess) { lg_set_error("matmul_tokens: %s", hipGetErrorString(e2)); rc = LG_ERR_HIP; }
         return rc;
+    }
+    if (at == LG_F16 && rsz != (uint32_t)n * 2u) {
+        lg_set_error("matmul_tokens: row bytes %u for %d values", rsz, n);
+        return LG_ERR_ARG;
     }
     /* workspace: quants, then scales for n/32 blocks (enough for either
      * form), the Q8_K bsums and the Q8_0 sums */
@@ -1597,7 +1606,8 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
     PfQ8K q = {};
     q.tld = tld;
     const size_t o_d = (size_t)tld * n, o_bs = o_d + (size_t)nb0 * tld * 4, o_as = o_bs + (size_t)tld * nb * 32;
-    const size_t bytes = o_as + (size_t)nb0 * tld * 4;
+    const size_t o_inv = lg_hsplit_bytes(T, n);   /* F16 form: the two parts, then a scale per token */
+    const size_t bytes = at == LG_F16 ? o_inv + (size_t)T * 4 : o_as + (size_t)nb0 * tld * 4;
     uint8_t* ws = nullptr;
     const hipError_t e = hipMalloc((void**)&ws, bytes);
     if (e != hipSuccess) { lg_set_error("matmul_tokens: hipMalloc(%zu): %s", bytes, hipGetErrorString(e)); return LG_ERR_NOMEM; }
@@ -1605,6 +1615,7 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
     q.d = (float*)(ws + o_d);
     q.bs = (int16_t*)(ws + o_bs);
     q.as = (int*)(ws + o_as);
+    if (at == LG_F16) q.hs = HSplit{(_Float16*)ws, (float*)(ws + o_inv)};
     int rc = lg_prefill_quantize(at, x, n, nullptr, 0.0f, n, T, q, (hipStream_t)stream);
     if (!rc) rc = lg_prefill_gemm(type, (const uint8_t*)w, rsz, d, n, q, T, out, d, 0, (hipStream_t)stream);
     const hipError_t e2 = hipStreamSynchronize((hipStream_t)stream);

@@ -1,0 +1,262 @@
+/* lg_fgemm.hip -- token GEMMs of F16 weights and fp32 activations on fp16
+ * MFMA: out[t][r] = W[r] . x[t] (dot_f16_f32, fast/lil_math.cpp:403-409, for
+ * many tokens at once).
+ *
+ * The fp32 MFMA multiplies at 157 TFLOP/s, the fp16 one at 2.5 PFLOP/s, and
+ * the weights are fp16 already: each activation goes in as two fp16 parts
+ * (HSplit in lg_fgemm.h: 22 bits of it), so x W = hi W + lo W with every
+ * product exact and fp32 accumulation.  Against 64 bits the sums come out
+ * closer than the fp32 MFMA's, whose longer chain of roundings weighs more
+ * than the two bits (see the test). */
+#include <math.h>
+
+#include <algorithm>
+
+#include "lg_common.h"
+#include "lg_fgemm.h"
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+
+/* token t = blockIdx.x: largest finite |x|, then the split row */
+__global__ __launch_bounds__(256) void k_hsplit(const float* __restrict__ x, int ldx, int K, HSplit o)
+{
+    __shared__ float s_m[4];
+    const int t = blockIdx.x, tid = threadIdx.x;
+    const float* xr = x + (size_t)t * ldx;
+    float m = 0.0f;
+    for (int i = 4 * tid; i < K; i += 1024) {
+        const float4 v = *(const float4*)(xr + i);
+        m = fmaxf(m, fmaxf(fmaxf(lg_finite_abs(v.x), lg_finite_abs(v.y)), fmaxf(lg_finite_abs(v.z), lg_finite_abs(v.w))));
+    }
+    m = lg_wave_max_nn(m);
+    if ((tid & 63) == 0) s_m[tid >> 6] = m;
+    __syncthreads();
+    const int k = lg_split_exp(fmaxf(fmaxf(s_m[0], s_m[1]), fmaxf(s_m[2], s_m[3])));
+    const float s = lg_pow2(k);
+    if (tid == 0) o.inv[t] = lg_pow2(-k);
+    for (int i = 4 * tid; i < K; i += 1024) {
+        const float4 f = *(const float4*)(xr + i);
+        const float v[4] = {f.x, f.y, f.z, f.w};
+        lg_split_store4(v, s, o, K, t, i);
+    }
+}
+
+int lg_hsplit(const float* x, int ldx, int K, int T, const HSplit& o, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_hsplit, dim3(T), dim3(256), 0, s, x, ldx, K, o);
+    return lg_check_launch("activation split");
+}
+
+/* A workgroup computes 32 MR WR weight rows x 32 MT WT tokens: WR x WT waves
+ * of MR x MT tiles of 32 x 32 (v_mfma_f32_32x32x16_f16, A = tokens, B =
+ * weight rows: lane l holds token / row l % 32, values 8 (l / 32) .. +7 of a
+ * 16-value step), and WK groups of such waves take consecutive parts of K
+ * with stages of their own, summed in group order through LDS at the end.
+ *
+ * Per step of 32 values both operands go through LDS, double-buffered, a
+ * step's loads in flight while the two steps before compute (one step ahead
+ * 240 instead of 229 us at 24576 x 4096, 500 tokens).  A row's 32 weights are four 16-byte pieces, a token's hi and lo
+ * eight; piece p of row or token j lies in the 1 KiB fragment (32 rows x 16
+ * values) it belongs to at lane slot 32 (p % 2) + (j ^ swz(p)): the 8
+ * threads that store a row's pieces hit 8 different 16-byte bank groups, and
+ * so do the lanes that read a fragment.
+ *
+ * What bounds it: 128 x 128 with 64 x 64 per wave reads 96 bytes of LDS a
+ * clock of the 128 possible at full MFMA rate and writes 48, so LDS holds it
+ * below ~70 % of that rate; 256 x 128 reads less but one workgroup of it a
+ * CU hides less of the loads' latency (267 against 229 us). */
+template <int MR, int MT, int WR, int WT, int WK, int EP>
+__global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_eu(2))) void k_hgemm(BGemm a, HSplit x)
+{
+    constexpr int TR = 32 * MR * WR, TT = 32 * MT * WT, NG = 64 * WR * WT;
+    constexpr int WB = TR * 64, XB = TT * 128, SB = WB + XB;   /* bytes of a stage */
+    constexpr int NW = TR * 4 / NG, NX = TT * 8 / NG;          /* pieces per thread */
+    static_assert(NW * NG == TR * 4 && NX * NG == TT * 8, "whole pieces");
+    static_assert((WK - 1) * TR * TT * 4 <= WK * 2 * SB || WK == 1, "the groups' sums fit the stages");
+    __shared__ __attribute__((aligned(16))) uint8_t s_st[WK][2][SB];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int kg = wave / (WR * WT), wr = wave % (WR * WT) / WT, wt = wave % WT, gt = threadIdx.x % NG;
+    const int h = lane >> 5, j = lane & 31;
+    const int nt = (a.T + TT - 1) / TT;
+    /* the token tiles of a row block on one XCD, 8 indices apart: its
+     * weights come from HBM once */
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int rb = (slot / nt) * 8 + xcd;
+    if (rb * TR >= a.R) return;   /* padding of the row blocks (whole workgroup) */
+    const int r0 = rb * TR, t0 = (slot % nt) * TT;
+    const int ns = a.K >> 5, nsg = (ns + WK - 1) / WK;
+    const int k0 = kg * nsg, kn = min(nsg, ns - k0);   /* this group's steps (kn may be <= 0) */
+
+    uint8_t(*st)[SB] = s_st[kg];
+    const uint8_t* wp[NW];
+    const uint8_t* xp[NX];
+    int ws[NW], xs[NX];
+#pragma unroll
+    for (int u = 0; u < NW; u++) {
+        const int q = gt + NG * u, r = q >> 2, p = q & 3;
+        wp[u] = a.w + (size_t)min(r0 + r, a.R - 1) * a.K * 2 + 16 * p;
+        ws[u] = ((r >> 5) * 2 + (p >> 1)) * 1024 + (32 * (p & 1) + ((r & 31) ^ (2 * p))) * 16;
+    }
+#pragma unroll
+    for (int u = 0; u < NX; u++) {
+        const int q = gt + NG * u, t = q >> 3, p = q & 7;
+        xp[u] = (const uint8_t*)x.h + (size_t)min(t0 + t, a.T - 1) * a.K * 4 + 16 * p;
+        xs[u] = WB + ((t >> 5) * 4 + (p >> 1)) * 1024 + (32 * (p & 1) + ((t & 31) ^ p)) * 16;
+    }
+    struct Stg {
+        v4i w[NW], x[NX];
+    };
+    auto load = [&](Stg& s, int i) __attribute__((always_inline)) {
+        const int k = max(min(k0 + i, ns - 1), 0);
+#pragma unroll
+        for (int u = 0; u < NW; u++) s.w[u] = *(const v4i*)(wp[u] + (size_t)k * 64);
+#pragma unroll
+        for (int u = 0; u < NX; u++) s.x[u] = *(const v4i*)(xp[u] + (size_t)k * 128);
+    };
+    auto store = [&](const Stg& s, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NW; u++) *(v4i*)(st[buf] + ws[u]) = s.w[u];
+#pragma unroll
+        for (int u = 0; u < NX; u++) *(v4i*)(st[buf] + xs[u]) = s.x[u];
+    };
+    v16f acc[MR][MT];
+#pragma unroll
+    for (int i = 0; i < MR; i++)
+#pragma unroll
+        for (int u = 0; u < MT; u++) acc[i][u] = (v16f){};
+    auto compute = [&](int buf) __attribute__((always_inline)) {
+        const uint8_t* sw = st[buf] + wr * MR * 2048;
+        const uint8_t* sx = st[buf] + WB + wt * MT * 4096;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            v8h wf[MR];
+#pragma unroll
+            for (int i = 0; i < MR; i++)
+                wf[i] = *(const v8h*)(sw + i * 2048 + s * 1024 + (32 * h + (j ^ (4 * s + 2 * h))) * 16);
+#pragma unroll
+            for (int u = 0; u < MT; u++) {
+#pragma unroll
+                for (int p = 0; p < 2; p++) {
+                    const v8h xf = *(const v8h*)(sx + u * 4096 + (2 * p + s) * 1024 + (32 * h + (j ^ (4 * p + 2 * s + h))) * 16);
+#pragma unroll
+                    for (int i = 0; i < MR; i++)
+                        acc[i][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf, wf[i], acc[i][u], 0, 0, 0);
+                }
+            }
+        }
+    };
+
+    Stg s0, s1;
+    load(s0, 0);
+    load(s1, 1);
+    store(s0, 0);
+    __syncthreads();
+    for (int i = 0; i < nsg; i += 2) {
+        load(s0, i + 2);
+        if (i < kn) compute(0);
+        store(s1, 1);
+        __syncthreads();
+        load(s1, i + 3);
+        if (i + 1 < kn) compute(1);
+        store(s0, 0);
+        __syncthreads();
+    }
+    if constexpr (WK > 1) {
+        /* the other groups' sums, in order (all stages are consumed) */
+        float* red = (float*)s_st;
+        constexpr int NR = MR * MT * 16;
+        if (kg) {
+#pragma unroll
+            for (int i = 0; i < MR; i++)
+#pragma unroll
+                for (int u = 0; u < MT; u++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) red[((kg - 1) * NR + (i * MT + u) * 16 + r) * NG + gt] = acc[i][u][r];
+        }
+        __syncthreads();
+        if (kg) return;
+#pragma unroll
+        for (int g = 0; g < WK - 1; g++)
+#pragma unroll
+            for (int i = 0; i < MR; i++)
+#pragma unroll
+                for (int u = 0; u < MT; u++)
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[i][u][r] += red[(g * NR + (i * MT + u) * 16 + r) * NG + gt];
+    }
+
+#pragma unroll
+    for (int u = 0; u < MT; u++) {
+        const int tb = t0 + (wt * MT + u) * 32 + 4 * h;   /* register r: token tb + 8 (r / 4) + r % 4 */
+        float inv[16];
+#pragma unroll
+        for (int r = 0; r < 16; r++) inv[r] = x.inv[min(tb + 8 * (r >> 2) + (r & 3), a.T - 1)];
+#pragma unroll
+        for (int i = 0; i < MR; i++) {
+            const int row = r0 + (wr * MR + i) * 32 + j;
+            if (row >= a.R) continue;
+            const float bias = EP <= EP_BIAS_GELU ? a.bias[row] : 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; r++) {
+                const int t = tb + 8 * (r >> 2) + (r & 3);
+                if (t >= a.T) continue;
+                float o = acc[i][u][r] * inv[r];
+                if constexpr (EP == EP_STORE) {
+                } else if constexpr (EP == EP_ADD) {
+                    o = a.out[(size_t)t * a.ldo + row] + o;
+                } else if constexpr (EP == EP_BIAS) {
+                    o = o + bias;
+                } else if constexpr (EP == EP_BIAS_RES) {
+                    o = o + (bias + a.res[(size_t)t * a.ldr + row]);
+                } else {
+                    /* gelu (fast/lil_math.cpp:978-984) of row + bias */
+                    const float g = o + bias;
+                    o = 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));
+                }
+                a.out[(size_t)t * a.ldo + row] = o;
+            }
+        }
+    }
+}
+
+template <int MR, int MT, int WR, int WT, int WK>
+static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
+{
+    const int nrb = ((a.R + 32 * MR * WR - 1) / (32 * MR * WR) + 7) & ~7, nt = (a.T + 32 * MT * WT - 1) / (32 * MT * WT);
+    const dim3 grid((unsigned)(nrb * nt)), blk(64 * WR * WT * WK);
+#define HG(E) hipLaunchKernelGGL((k_hgemm<MR, MT, WR, WT, WK, E>), grid, blk, 0, s, a, x)
+    switch (ep) {
+    case EP_BIAS: HG(EP_BIAS); break;
+    case EP_BIAS_RES: HG(EP_BIAS_RES); break;
+    case EP_BIAS_GELU: HG(EP_BIAS_GELU); break;
+    case EP_ADD: HG(EP_ADD); break;
+    default: HG(EP_STORE); break;
+    }
+#undef HG
+}
+
+/* The tile by how many workgroups it gives the 256 CUs (us at that tile /
+ * the next candidates, weights cycled through more than the caches hold):
+ * 128 x 128 while it fills them -- 24576 x 4096, 500 tokens 229 (881 TFLOP/s
+ * of the two products; 256 x 128 267, 128 x 64 264), 1152 x 384, 4096 tokens
+ * 21 -- then 128 x 64 (24576 x 4096, 150 tokens 117 / 129), with K in two
+ * parts where a CU would hold one workgroup only (4096 x 4096, 500 tokens 50
+ * / 54 unsplit), then 64 x 64 (384 x 1536, 4096 tokens 32 / 35; split:
+ * 4096 x 4096, 150 tokens 32 / 34), and 32 x 32 with K in four parts for the
+ * smallest (384 x 1536, 512 tokens 8.4 / 13) and for up to 32 tokens, where
+ * the weights' stream is the bound (24576 x 4096, 13 tokens 50, 4.1 TB/s;
+ * 64 x 64 60). */
+int lg_hgemm(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
+{
+    auto wgs = [&](int tr, int tt) { return (long)((a.R + tr - 1) / tr) * ((a.T + tt - 1) / tt); };
+    if (a.T <= 32) hgemm_launch<1, 1, 1, 1, 4>(a, x, ep, s);
+    else if (wgs(128, 128) >= 256) hgemm_launch<2, 2, 2, 2, 1>(a, x, ep, s);
+    else if (wgs(128, 64) >= 384) hgemm_launch<2, 1, 2, 2, 1>(a, x, ep, s);
+    else if (wgs(128, 64) >= 224) hgemm_launch<2, 1, 2, 2, 2>(a, x, ep, s);
+    else if (wgs(64, 64) >= 320) hgemm_launch<1, 1, 2, 2, 1>(a, x, ep, s);
+    else if (wgs(64, 64) >= 128) hgemm_launch<1, 1, 2, 2, 2>(a, x, ep, s);
+    else hgemm_launch<1, 1, 1, 1, 4>(a, x, ep, s);
+    return lg_check_launch("fp16 gemm");
+}

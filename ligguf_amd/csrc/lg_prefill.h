@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lg_fgemm.h"
+
 /* Quantized activations of T tokens, structure of arrays (the GEMMs stage a
  * token tile with 16-byte loads).  Q8_K form (K-quant weights): qs [T][K]
  * int8, d [K/256][tld] block scales (tokens contiguous), bs [T][K/256][16]
@@ -16,7 +18,8 @@ struct PfQ8K {
     int16_t* bs;
     int* as;
     int tld;
-    float* f;        /* F32 form (F32/F16 weights): the fp32 activations [T][K], nothing quantized */
+    float* f;        /* F32 form (F32 weights): the fp32 activations [T][K], nothing quantized */
+    HSplit hs;       /* F16 form (F16 weights): the fp32 activations as two fp16 parts */
 };
 
 /* one weight matrix as the prefill reads it: GGUF rows of `type` */
@@ -59,14 +62,16 @@ struct PfBuffers {
     PfQ8K qk;        /* Q8_K form, width up to n_ff (qs NULL when no matrix takes it) */
     PfQ8K q0;        /* Q8_0 form (likewise) */
     PfQ8K qf;        /* F32 form (likewise; only f and tld) */
+    PfQ8K qh;        /* F16 form (likewise; only hs and tld) */
     /* activation trace of one pass (NULL: none): token t's activation k in
      * block_q8_K / block_q8_0 rows at trace + (t (4 L + 1) + k) stride */
     uint8_t* trace;
     size_t trace_stride;
 };
 
-/* activation form a weight type takes: LG_Q8_K, LG_Q8_0, LG_F32 (F32/F16
- * weights), or -1 when the batched GEMMs do not take the type */
+/* activation form a weight type takes: LG_Q8_K, LG_Q8_0, LG_F32 (F32
+ * weights), LG_F16 (F16 weights: fp32 values in two fp16 parts), or -1 when
+ * the batched GEMMs do not take the type */
 int lg_prefill_act_type(int wtype);
 
 /* the prefill attention's head widths and query heads per KV head */
@@ -87,11 +92,11 @@ int lg_prefill_gemm(int wtype, const uint8_t* W, uint32_t rsz, int rows, int col
 bool lg_prefill_gemm16();
 /* rmsnorm (norm_w != NULL) and the activation quantizer of qtype (LG_Q8_K,
  * n a multiple of 256, or LG_Q8_0, n a multiple of 32; LG_F32: the fp32
- * values into q.f) for T tokens of width n */
+ * values into q.f, LG_F16: into q.hs) for T tokens of width n */
 int lg_prefill_quantize(int qtype, const float* x, int ldx, const float* norm_w, float eps, int n, int T,
                         const PfQ8K& q, hipStream_t s);
 
-/* F32/F16 weights x fp32 activations on fp32 MFMA (lg_bert.hip's token
- * GEMM): out[t][r] (+)= W[r] . x[t] */
-int lg_fgemm_tokens(int wtype, const uint8_t* W, int rows, int cols, const float* x, int ldx, int T, float* out, int ldo,
+/* F32 weights x fp32 activations on fp32 MFMA (lg_bert.hip's token GEMM):
+ * out[t][r] (+)= W[r] . x[t] */
+int lg_fgemm_tokens(const uint8_t* W, int rows, int cols, const float* x, int ldx, int T, float* out, int ldo,
                     int accumulate, hipStream_t s);

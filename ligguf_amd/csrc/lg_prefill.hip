@@ -84,10 +84,28 @@ __device__ __forceinline__ void pf_store(const float v[4], const PfQ8K& q, int n
     if constexpr (QT == LG_Q8_K) pf_store_q8k(v, q, n, t, b);
     else if constexpr (QT == LG_Q8_0) pf_store_q8_0(v, q, n, t, b);
     else {
-        /* the fp32 values (F32/F16 weights take them unquantized) */
+        /* the fp32 values (F32 weights take them unquantized) */
         const int i = b * 256 + 4 * (threadIdx.x & 63);
         if (i < n) *(float4*)(q.f + (size_t)t * n + i) = make_float4(v[0], v[1], v[2], v[3]);
     }
+}
+
+__device__ __forceinline__ float pf_amax(const float v[4], float m)
+{
+#pragma unroll
+    for (int j = 0; j < 4; j++) m = fmaxf(m, lg_finite_abs(v[j]));
+    return m;
+}
+
+/* the token's split exponent from its 4 waves' largest values (red: 4 floats
+ * of LDS, which earlier reads may still hold) */
+__device__ __forceinline__ int pf_token_exp(float m, float* red)
+{
+    m = lg_wave_max_nn(m);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    return lg_split_exp(fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
 }
 
 /* token t (one workgroup of 4 waves): rmsnorm(x_t) * w (w != NULL) or
@@ -117,16 +135,36 @@ __global__ __launch_bounds__(256) void k_pf_quant(const float* __restrict__ x, i
         scale = 1.0f / sqrtf(ss / (float)n + eps);
     }
     const int nb = (n + 255) / 256;
-    for (int b = wave; b < nb; b += 4) {
+    auto value = [&](int b, float (&v)[4]) {
         const int base = b * 256 + 4 * lane;
         const bool in = base < n;   /* Q8_0 widths that are no multiple of 256: zeros past the end, not stored */
         const float4 tv = in ? *(const float4*)(xr + base) : make_float4(0.f, 0.f, 0.f, 0.f);
-        float v[4] = {tv.x, tv.y, tv.z, tv.w};
+        v[0] = tv.x; v[1] = tv.y; v[2] = tv.z; v[3] = tv.w;
         if (w && in) {
             const float4 g = *(const float4*)(w + base);
             v[0] = tv.x * scale * g.x; v[1] = tv.y * scale * g.y; v[2] = tv.z * scale * g.z; v[3] = tv.w * scale * g.w;
         }
-        pf_store<QT>(v, q, n, t, b);
+    };
+    float v[4];
+    if constexpr (QT == LG_F16) {
+        /* the token's scale first: its values again for the split (they are in L1 / L2) */
+        float m = 0.0f;
+        for (int b = wave; b < nb; b += 4) {
+            value(b, v);
+            m = pf_amax(v, m);
+        }
+        const int k = pf_token_exp(m, s_ss);
+        if (threadIdx.x == 0) q.hs.inv[t] = lg_pow2(-k);
+        for (int b = wave; b < nb; b += 4) {
+            value(b, v);
+            const int i = b * 256 + 4 * lane;
+            if (i < n) lg_split_store4(v, lg_pow2(k), q.hs, n, t, i);
+        }
+    } else {
+        for (int b = wave; b < nb; b += 4) {
+            value(b, v);
+            pf_store<QT>(v, q, n, t, b);
+        }
     }
 }
 
@@ -147,6 +185,33 @@ __global__ __launch_bounds__(64) void k_pf_swiglu_quant(const float* __restrict_
     v[2] = (g.z / (1.0f + expf(-g.z))) * u.z;
     v[3] = (g.w / (1.0f + expf(-g.w))) * u.w;
     pf_store<QT>(v, q, nff, t, b);
+}
+
+/* the same of token t (one workgroup) into two fp16 parts: the values go
+ * back into the row's up half until the token's scale is known */
+__global__ __launch_bounds__(256) void k_pf_swiglu_split(float* __restrict__ ug, int nff, PfQ8K q)
+{
+    __shared__ float s_m[4];
+    const int t = blockIdx.x;
+    float* ur = ug + (size_t)t * 2 * nff;
+    float m = 0.0f;
+    for (int i = 4 * threadIdx.x; i < nff; i += 1024) {
+        const float4 u = *(const float4*)(ur + i), g = *(const float4*)(ur + nff + i);
+        float v[4];
+        v[0] = (g.x / (1.0f + expf(-g.x))) * u.x;
+        v[1] = (g.y / (1.0f + expf(-g.y))) * u.y;
+        v[2] = (g.z / (1.0f + expf(-g.z))) * u.z;
+        v[3] = (g.w / (1.0f + expf(-g.w))) * u.w;
+        m = pf_amax(v, m);
+        *(float4*)(ur + i) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+    const int k = pf_token_exp(m, s_m);
+    if (threadIdx.x == 0) q.hs.inv[t] = lg_pow2(-k);
+    for (int i = 4 * threadIdx.x; i < nff; i += 1024) {   /* each thread its own values */
+        const float4 f = *(const float4*)(ur + i);
+        const float v[4] = {f.x, f.y, f.z, f.w};
+        lg_split_store4(v, lg_pow2(k), q.hs, nff, t, i);
+    }
 }
 
 /* QK-norm + RoPE + KV rows of token t at position pos0 + t */
@@ -928,14 +993,16 @@ static int gemm_q4k(const uint8_t* W, uint32_t rsz, int rows, int cols, const Pf
 int lg_prefill_quantize(int qtype, const float* x, int ldx, const float* norm_w, float eps, int n, int T,
                         const PfQ8K& q, hipStream_t s)
 {
-    if (!x || !(qtype == LG_F32 ? (void*)q.f : (void*)q.qs) || n <= 0 || n % (qtype == LG_Q8_K ? 256 : 32) ||
-        T <= 0 || T > q.tld || ldx < n || (qtype != LG_Q8_K && qtype != LG_Q8_0 && qtype != LG_F32)) {
+    const void* dst = qtype == LG_F32 ? (void*)q.f : qtype == LG_F16 ? (void*)q.hs.h : (void*)q.qs;
+    if (!x || !dst || n <= 0 || n % (qtype == LG_Q8_K ? 256 : 32) || T <= 0 || T > q.tld || ldx < n ||
+        (qtype != LG_Q8_K && qtype != LG_Q8_0 && qtype != LG_F32 && qtype != LG_F16)) {
         lg_set_error("prefill quantize: bad arguments (type %d, n %d, T %d)", qtype, n, T);
         return LG_ERR_ARG;
     }
     const dim3 grid(T), blk(256);
     if (qtype == LG_Q8_K) hipLaunchKernelGGL(k_pf_quant<LG_Q8_K>, grid, blk, 0, s, x, ldx, norm_w, eps, n, q);
     else if (qtype == LG_Q8_0) hipLaunchKernelGGL(k_pf_quant<LG_Q8_0>, grid, blk, 0, s, x, ldx, norm_w, eps, n, q);
+    else if (qtype == LG_F16) hipLaunchKernelGGL(k_pf_quant<LG_F16>, grid, blk, 0, s, x, ldx, norm_w, eps, n, q);
     else hipLaunchKernelGGL(k_pf_quant<LG_F32>, grid, blk, 0, s, x, ldx, norm_w, eps, n, q);
     return lg_check_launch("prefill quantize");
 }
@@ -1835,7 +1902,8 @@ int lg_prefill_act_type(int wtype)
     switch (wtype) {
     case LG_Q2_K: case LG_Q3_K: case LG_Q4_K: case LG_Q5_K: case LG_Q6_K: case LG_Q6_K_R: return LG_Q8_K;
     case LG_Q8_0: case LG_Q1_0: case LG_Q1_G: case LG_Q8_0_R: case LG_Q1_0_R: case LG_Q1_G_R: return LG_Q8_0;
-    case LG_F32: case LG_F16: return LG_F32;
+    case LG_F32: return LG_F32;
+    case LG_F16: return LG_F16;
     default: return -1;
     }
 }
@@ -1871,12 +1939,17 @@ int lg_prefill_gemm(int wtype, const uint8_t* W, uint32_t rsz, int rows, int col
         return LG_ERR_TYPE;
     }
     const int64_t rb = pf_row_bytes(wtype, cols);
-    if (at == LG_F32) {
-        if (rb < 0 || rsz != (uint32_t)rb || !x.f || T > x.tld) {
-            lg_set_error("prefill gemm: bad arguments (type %d, cols %d, row bytes %u, T %d)", wtype, cols, rsz, T);
+    if (at == LG_F32 || at == LG_F16) {
+        if (rb < 0 || rsz != (uint32_t)rb || !(at == LG_F32 ? (void*)x.f : (void*)x.hs.h) || T > x.tld || !W || !out ||
+            rows <= 0 || cols < 32 || T <= 0 || ldo < rows) {
+            lg_set_error("prefill gemm: bad arguments (type %d, rows %d, cols %d, row bytes %u, T %d)", wtype, rows, cols,
+                         rsz, T);
             return LG_ERR_ARG;
         }
-        return lg_fgemm_tokens(wtype, W, rows, cols, x.f, cols, T, out, ldo, accumulate, s);
+        if (at == LG_F32) return lg_fgemm_tokens(W, rows, cols, x.f, cols, T, out, ldo, accumulate, s);
+        BGemm a = {};
+        a.w = W; a.R = rows; a.K = cols; a.T = T; a.out = out; a.ldo = ldo;
+        return lg_hgemm(a, x.hs, accumulate ? EP_ADD : EP_STORE, s);
     }
     if (!W || !out || !x.qs || !x.d || (at == LG_Q8_K && !x.bs) || (wtype == LG_Q1_G && !x.as) || rows <= 0 ||
         cols < 32 || rb < 0 || rsz != (uint32_t)rb || T <= 0 || T > x.tld || x.tld % 4 || ldo < rows) {
@@ -2224,10 +2297,10 @@ int lg_prefill_layers(const PfModel& M, PfBuffers& B, int T, int pos0, hipStream
     }
     const int ne = M.n_embed, kvd = M.kv_dim, qs = ne + 2 * kvd, nff = M.n_ff;
     const size_t tstride = (size_t)(4 * M.n_layers + 1) * B.trace_stride;
-    /* activation forms the matrices take: bit 0 Q8_K, bit 1 Q8_0, bit 2 F32 */
+    /* activation forms the matrices take: bit 0 Q8_K, bit 1 Q8_0, bit 2 F32, bit 3 F16 */
     auto fam = [](const PfMat& W) {
         const int at = lg_prefill_act_type(W.type);
-        return at == LG_Q8_K ? 1 : at == LG_Q8_0 ? 2 : 4;
+        return at == LG_Q8_K ? 1 : at == LG_Q8_0 ? 2 : at == LG_F32 ? 4 : 8;
     };
     auto trace = [&](int f, int n, int k) -> int {
         if (!B.trace || !(f & 3)) return LG_OK;   /* fp32 activations are not quantized: nothing to record */
@@ -2243,11 +2316,12 @@ int lg_prefill_layers(const PfModel& M, PfBuffers& B, int T, int pos0, hipStream
         if ((f & 1) && (rc = lg_prefill_quantize(LG_Q8_K, x, n, w, M.eps, n, T, B.qk, s))) return rc;
         if ((f & 2) && (rc = lg_prefill_quantize(LG_Q8_0, x, n, w, M.eps, n, T, B.q0, s))) return rc;
         if ((f & 4) && (rc = lg_prefill_quantize(LG_F32, x, n, w, M.eps, n, T, B.qf, s))) return rc;
+        if ((f & 8) && (rc = lg_prefill_quantize(LG_F16, x, n, w, M.eps, n, T, B.qh, s))) return rc;
         return trace(f, n, k);
     };
     auto gemm = [&](const PfMat& W, int cols, float* o, int ldo, int acc) {
         const int f = fam(W);
-        return lg_prefill_gemm(W.type, W.w, W.rsz, W.rows, cols, f == 1 ? B.qk : f == 2 ? B.q0 : B.qf, T, o, ldo, acc, s);
+        return lg_prefill_gemm(W.type, W.w, W.rsz, W.rows, cols, f == 1 ? B.qk : f == 2 ? B.q0 : f == 4 ? B.qf : B.qh, T, o, ldo, acc, s);
     };
     int rc;
     hipLaunchKernelGGL(k_pf_embed, dim3(T), dim3(256), 0, s, M.embd_t, M.embd, M.embd_rsz, B.toks, ne, B.x);
@@ -2286,7 +2360,8 @@ int lg_prefill_layers(const PfModel& M, PfBuffers& B, int T, int pos0, hipStream
         const dim3 sg((nff + 255) / 256, T);
         if (f_d == 1) hipLaunchKernelGGL(k_pf_swiglu_quant<LG_Q8_K>, sg, dim3(64), 0, s, B.ug, nff, B.qk);
         else if (f_d == 2) hipLaunchKernelGGL(k_pf_swiglu_quant<LG_Q8_0>, sg, dim3(64), 0, s, B.ug, nff, B.q0);
-        else hipLaunchKernelGGL(k_pf_swiglu_quant<LG_F32>, sg, dim3(64), 0, s, B.ug, nff, B.qf);
+        else if (f_d == 4) hipLaunchKernelGGL(k_pf_swiglu_quant<LG_F32>, sg, dim3(64), 0, s, B.ug, nff, B.qf);
+        else hipLaunchKernelGGL(k_pf_swiglu_split, dim3(T), dim3(256), 0, s, B.ug, nff, B.qh);
         if ((rc = lg_check_launch("prefill swiglu"))) return rc;
         if ((rc = trace(f_d, nff, 4 * l + 3))) return rc;
         if ((rc = gemm(L.down, nff, B.x, ne, 1))) return rc;
