@@ -26,6 +26,7 @@
 #include "lg_rope.h"
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned short v2u16 __attribute__((ext_vector_type(2)));
 typedef short v2i16 __attribute__((ext_vector_type(2)));
@@ -435,9 +436,8 @@ __global__ __launch_bounds__(PF_NT) __attribute__((amdgpu_waves_per_eu(4))) void
 /* The same products on the 32 x 32 forms: v_mfma_i32_32x32x32_i8 takes 16
  * bytes of a 32-row A and of a 32-column B per lane, twice the multiplies
  * of a 16x16x64 product per operand byte, so each token fragment read from
- * LDS feeds twice the work.  A workgroup of 4 waves computes 128 rows x 64
- * tokens, a wave 32 rows x 64 tokens (two 32 x 32 tiles, token rows i,
- * weight columns j): lane l holds row j = l % 32 of its wave's rows and the
+ * LDS feeds twice the work.  A wave computes 32 rows x 64 or 32 tokens (32 x
+ * 32 tiles, token rows i, weight columns j): lane l holds row j = l % 32 of its wave's rows and the
  * K bytes 16 (l / 32) .. +15 of a 32-value sub-block -- sub-block 2c is the
  * low nibbles and 2c+1 the high nibbles of the same 16 bytes of qs --
  * against the token's quants 32s + 16 (l / 32) .. +15, read from its LDS
@@ -470,15 +470,13 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-#define PF2_NT 256
-#define PF2_RB 128    /* rows per workgroup */
 #define PF2_AST 272   /* LDS row stride of a token's 256 quants */
-/* KS = 2 (the 4096-row att_out and down products, whose 128 x 64 tiles
- * alone would leave one wave per SIMD): 8 waves, waves 4..7 take the second
- * half of K with LDS stages of their own, and their sums are added to the
- * first half's through LDS at the end (acc0 + acc1, one fixed order) */
-template <int WT, int ACC, int KS>
-__global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_gemm_k32(
+/* A workgroup of RW x KS waves computes 32 RW rows x TT tokens: RW waves of
+ * 32 rows side by side, and KS groups of them that take consecutive parts of
+ * K with LDS stages of their own; the parts' sums are added in order through
+ * LDS at the end (acc0 + acc1 + ..) */
+template <int WT, int ACC, int RW, int KS, int TT>
+__global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_gemm_k32(
     const uint8_t* __restrict__ W, uint32_t rsz, int R, int K, PfQ8K x, int T, float* __restrict__ out, int ldo)
 {
     static_assert(WT == LG_Q2_K || WT == LG_Q3_K || WT == LG_Q4_K || WT == LG_Q5_K || WT == LG_Q6_K || WT == LG_Q6_K_R,
@@ -491,72 +489,85 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
     constexpr bool MINS = MK != 0;
     constexpr int BSZ = WT == LG_Q2_K ? LG_BS_Q2_K : WT == LG_Q3_K ? LG_BS_Q3_K : WT == LG_Q4_K ? LG_BS_Q4_K
                       : WT == LG_Q5_K ? LG_BS_Q5_K : LG_BS_Q6_K;
-    constexpr int TT = 64;   /* tokens per workgroup: two 32-token tiles per wave */
+    constexpr int NTL = TT / 32;        /* 32-token tiles per wave */
+    constexpr int NG = 64 * RW;         /* threads of a K part */
+    constexpr int NA = TT * 16 / NG;    /* 16-byte quant pieces per thread and stage */
+    constexpr int NB = (TT * 4 + NG - 1) / NG;   /* bsums pieces */
+    static_assert(NA * NG == TT * 16 && NG >= TT, "stage pieces");
     __shared__ __attribute__((aligned(16))) int8_t s_a[KS][2][TT * PF2_AST];
     /* per token: p_hi[8], p_lo[8] or the 16 bsums (the mins term) */
     constexpr int MST = MINS ? TT * 16 : 8;
     __shared__ __attribute__((aligned(16))) _Float16 s_m[KS][2][MST];
     __shared__ __attribute__((aligned(16))) float s_d[KS][2][TT];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kh = wave >> 2, tid = threadIdx.x & (PF2_NT - 1);   /* K half; thread within it */
+    const int kh = wave / RW, tid = threadIdx.x % NG;   /* K part; thread within it */
     const int h = lane >> 5, j = lane & 31;
     const int nb = K >> 8;
-    /* this half's blocks b0 .. b0 + nbh - 1; every wave runs L steps */
-    const int nb0 = KS == 2 ? (nb + 1) / 2 : nb;
-    const int b0 = kh * nb0, nbh = kh ? nb - nb0 : nb0, L = nb0;
+    /* this part's blocks b0 .. b0 + nbh - 1 (nbh may be <= 0); every wave runs L steps */
+    const int L = (nb + KS - 1) / KS;
+    const int b0 = kh * L, nbh = min(L, nb - b0);
     const int nt = (T + TT - 1) / TT;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int rb = (slot / nt) * 8 + xcd;
-    if (rb * PF2_RB >= R) return;   /* padding of the row blocks to a multiple of 8 (whole workgroup) */
+    if (rb * 32 * RW >= R) return;   /* padding of the row blocks to a multiple of 8 (whole workgroup) */
     const int t0 = (slot % nt) * TT;
-    const int row = rb * PF2_RB + (wave & 3) * 32 + j;
+    const int row = (rb * RW + wave % RW) * 32 + j;
     const uint8_t* wr = W + (size_t)min(row, R - 1) * rsz;
     int8_t(*sa_)[TT * PF2_AST] = s_a[kh];
     _Float16(*sm_)[MST] = s_m[kh];
     float(*sd_)[TT] = s_d[kh];
 
-    /* staging, per block: quant chunk q = tid + 256 u (token q / 16, piece
-     * q % 16); thread tid also takes bsums 4 (tid % 4) .. +3 of token tid / 4
-     * (pair sums 2 (tid % 4), +1) and, tid < 64, the d of token tid */
+    /* staging, per block: quant piece q = tid + NG u (token q / 16, piece
+     * q % 16); bsums piece q = tid + NG u (token q / 4, bsums 4 (q % 4) ..
+     * +3, pair sums 2 (q % 4), +1); tid < TT the d of token tid */
     struct Stg {   /* clang vectors, not HIP's uint4 structs: their copies stay in registers */
-        v4i a[4];
-        uint2 bs;
+        v4i a[NA];
+        v2u bs[NB];
         float d;
     };
     auto stage_load = [&](Stg& st, int b) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int q = tid + PF2_NT * u, tok = min(t0 + (q >> 4), T - 1);
+        for (int u = 0; u < NA; u++) {
+            const int q = tid + NG * u, tok = min(t0 + (q >> 4), T - 1);
             st.a[u] = *(const v4i*)(x.qs + (size_t)tok * K + (size_t)b * 256 + (q & 15) * 16);
         }
         if constexpr (MINS) {   /* the bsums feed the mins term */
-            const int tb = min(t0 + (tid >> 2), T - 1);
-            st.bs = *(const uint2*)(x.bs + ((size_t)tb * nb + b) * 16 + (tid & 3) * 4);
+#pragma unroll
+            for (int u = 0; u < NB; u++) {
+                const int q = tid + NG * u, tb = min(t0 + (q >> 2), T - 1);
+                st.bs[u] = *(const v2u*)(x.bs + ((size_t)tb * nb + b) * 16 + (q & 3) * 4);
+            }
         }
-        st.d = x.d[(size_t)b * x.tld + min(t0 + (tid & 63), x.tld - 1)];
+        st.d = x.d[(size_t)b * x.tld + min(t0 + tid % TT, x.tld - 1)];
     };
     auto stage_store = [&](const Stg& st, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int q = tid + PF2_NT * u;
+        for (int u = 0; u < NA; u++) {
+            const int q = tid + NG * u;
             *(v4i*)(sa_[buf] + (q >> 4) * PF2_AST + (q & 15) * 16) = st.a[u];
         }
-        const int tok = tid >> 2;   /* bsums / mins of token tid / 4 */
-        if constexpr (MK == 2) {
-            const v4h m = {(_Float16)(float)(int16_t)(st.bs.x & 0xffff), (_Float16)(float)(int16_t)(st.bs.x >> 16),
-                           (_Float16)(float)(int16_t)(st.bs.y & 0xffff), (_Float16)(float)(int16_t)(st.bs.y >> 16)};
-            *(v4h*)(sm_[buf] + tok * 16 + 4 * (tid & 3)) = m;
-        } else if constexpr (MINS) {
-            const int s0 = 2 * (tid & 3);
-            const int p0 = (int)(int16_t)(st.bs.x & 0xffff) + (int)(int16_t)(st.bs.x >> 16);
-            const int p1 = (int)(int16_t)(st.bs.y & 0xffff) + (int)(int16_t)(st.bs.y >> 16);
-            _Float16* m = sm_[buf] + tok * 16;
-            m[s0] = (_Float16)(float)(p0 >> 6);
-            m[s0 + 1] = (_Float16)(float)(p1 >> 6);
-            m[8 + s0] = (_Float16)(float)(p0 & 63);
-            m[8 + s0 + 1] = (_Float16)(float)(p1 & 63);
+        if constexpr (MINS) {
+#pragma unroll
+            for (int u = 0; u < NB; u++) {
+                const int q = tid + NG * u, tok = q >> 2;
+                if (NB * NG != TT * 4 && tok >= TT) break;
+                if constexpr (MK == 2) {
+                    const v4h m = {(_Float16)(float)(int16_t)(st.bs[u][0] & 0xffff), (_Float16)(float)(int16_t)(st.bs[u][0] >> 16),
+                                   (_Float16)(float)(int16_t)(st.bs[u][1] & 0xffff), (_Float16)(float)(int16_t)(st.bs[u][1] >> 16)};
+                    *(v4h*)(sm_[buf] + tok * 16 + 4 * (q & 3)) = m;
+                } else {
+                    const int s0 = 2 * (q & 3);
+                    const int p0 = (int)(int16_t)(st.bs[u][0] & 0xffff) + (int)(int16_t)(st.bs[u][0] >> 16);
+                    const int p1 = (int)(int16_t)(st.bs[u][1] & 0xffff) + (int)(int16_t)(st.bs[u][1] >> 16);
+                    _Float16* m = sm_[buf] + tok * 16;
+                    m[s0] = (_Float16)(float)(p0 >> 6);
+                    m[s0 + 1] = (_Float16)(float)(p1 >> 6);
+                    m[8 + s0] = (_Float16)(float)(p0 & 63);
+                    m[8 + s0 + 1] = (_Float16)(float)(p1 & 63);
+                }
+            }
         }
-        if (tid < 64) sd_[buf][tid] = st.d;
+        if (tid < TT) sd_[buf][tid] = st.d;
     };
     /* the lane's weight bytes of one block: Q4_K the header and 4 x 16 B of
      * qs; Q6_K 4 x 16 B of ql, 2 x 16 B of qh, the 16 scales and d */
@@ -638,15 +649,15 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         }
     };
 
-    v16f acc[2];
-    acc[0] = (v16f){};
-    acc[1] = (v16f){};
+    v16f acc[NTL];
+#pragma unroll
+    for (int t = 0; t < NTL; t++) acc[t] = (v16f){};
 
     auto compute6 = [&](int buf, const Blk6& cur) __attribute__((always_inline)) {
         const float dw = lg_h2f((uint16_t)cur.d);
-        v16i Sh[2], Sl[2];
+        v16i Sh[NTL], Sl[NTL];
 #pragma unroll
-        for (int t = 0; t < 2; t++) Sh[t] = Sl[t] = (v16i){};
+        for (int t = 0; t < NTL; t++) Sh[t] = Sl[t] = (v16i){};
         const int8_t* sa = sa_[buf] + j * PF2_AST + 16 * h;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
@@ -673,7 +684,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
                 bl[k] = (int)(__builtin_amdgcn_perm(lg_bits<uint32_t>(wo), lg_bits<uint32_t>(we), 0x06020400u) & 0x3F3F3F3Fu);
             }
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < NTL; t++) {
                 const uint4 a = *(const uint4*)(sa + 32 * t * PF2_AST + 32 * s);
                 const v4i af = {(int)a.x, (int)a.y, (int)a.z, (int)a.w};
                 Sh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bh, Sh[t], 0, 0, 0);
@@ -681,7 +692,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
             const v16i S = Sh[t] * 64 + Sl[t];
 #pragma unroll
             for (int g = 0; g < 4; g++) {
@@ -703,9 +714,9 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         v8h bm;   /* mins of sub-blocks 8h .. 8h + 7 */
 #pragma unroll
         for (int k = 0; k < 8; k++) bm[k] = (_Float16)(float)(((uint32_t)cur.sc[2 * h + (k >> 2)] >> (8 * (k & 3) + 4)) & 15u);
-        v16i S[2];
+        v16i S[NTL];
 #pragma unroll
-        for (int t = 0; t < 2; t++) S[t] = (v16i){};
+        for (int t = 0; t < NTL; t++) S[t] = (v16i){};
         const int8_t* sa = sa_[buf] + j * PF2_AST + 16 * h;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
@@ -717,14 +728,14 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             for (int k = 0; k < 4; k++)
                 bw[k] = (int)lg_bits<uint32_t>(lg_bits<v2u16>(((uint32_t)cur.qs[n][k] >> (2 * jj)) & 0x03030303u) * sc2);
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < NTL; t++) {
                 const uint4 a = *(const uint4*)(sa + 32 * t * PF2_AST + 32 * s);
                 const v4i af = {(int)a.x, (int)a.y, (int)a.z, (int)a.w};
                 S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bw, S[t], 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
             const v8h am = *(const v8h*)(sm_[buf] + (32 * t + j) * 16 + 8 * h);
             const v16f M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, (v16f){}, 0, 0, 0);
 #pragma unroll
@@ -744,9 +755,9 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
      * reaches 128), one product per chunk and S = -S' */
     auto compute3 = [&](int buf, const Blk3& cur) __attribute__((always_inline)) {
         const float dw = lg_h2f((uint16_t)cur.d);
-        v16i S[2];
+        v16i S[NTL];
 #pragma unroll
-        for (int t = 0; t < 2; t++) S[t] = (v16i){};
+        for (int t = 0; t < NTL; t++) S[t] = (v16i){};
         const int8_t* sa = sa_[buf] + j * PF2_AST + 16 * h;
 #pragma unroll
         for (int s = 0; s < 8; s++) {
@@ -769,14 +780,14 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
                 bw[k] = (int)__builtin_amdgcn_perm(lg_bits<uint32_t>(wo), lg_bits<uint32_t>(we), 0x06020400u);
             }
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < NTL; t++) {
                 const uint4 a = *(const uint4*)(sa + 32 * t * PF2_AST + 32 * s);
                 const v4i af = {(int)a.x, (int)a.y, (int)a.z, (int)a.w};
                 S[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bw, S[t], 0, 0, 0);
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
 #pragma unroll
             for (int g = 0; g < 4; g++) {
                 const float4 dx = *(const float4*)(sd_[buf] + 32 * t + 8 * g + 4 * h);
@@ -809,9 +820,9 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             const int m = (int)((mn[s >> 2] >> (8 * (s & 3))) & 0xFFu);
             bm[s] = (_Float16)(float)(h ? m : 64 * m);
         }
-        v16i Sh[2], Sl[2];
+        v16i Sh[NTL], Sl[NTL];
 #pragma unroll
-        for (int t = 0; t < 2; t++) Sh[t] = Sl[t] = (v16i){};
+        for (int t = 0; t < NTL; t++) Sh[t] = Sl[t] = (v16i){};
         const int8_t* sa = sa_[buf] + j * PF2_AST + 16 * h;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -847,7 +858,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
                     }
                 }
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
+                for (int t = 0; t < NTL; t++) {
                     const uint4 a = *(const uint4*)(sa + 32 * t * PF2_AST + 32 * s);
                     const v4i af = {(int)a.x, (int)a.y, (int)a.z, (int)a.w};
                     Sh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bh, Sh[t], 0, 0, 0);
@@ -856,7 +867,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             }
         }
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
             const v8h am = *(const v8h*)(sm_[buf] + (32 * t + j) * 16 + 8 * h);
             const v16f M = __builtin_amdgcn_mfma_f32_32x32x16_f16(am, bm, (v16f){}, 0, 0, 0);
             const v16i S = Sh[t] * (WT == LG_Q4_K ? 8 : 64) + Sl[t];
@@ -874,10 +885,10 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
       }
     };
 
-    /* step i of this half: the token tile of block b0 + i + 2 loads into
+    /* step i of this part: the token tile of block b0 + i + 2 loads into
      * registers while block b0 + i computes, and goes to LDS after it (two
      * blocks' compute for each staging load; one for the weights) */
-    auto blk = [&](int i) { return b0 + min(i, nbh - 1); };
+    auto blk = [&](int i) { return min(b0 + max(min(i, nbh - 1), 0), nb - 1); };
     Blk cur, nxt;
     Stg st0, st1;
     stage_load(st0, blk(0));
@@ -895,31 +906,34 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         __syncthreads();                          \
     } while (0)
     /* pairs of steps (an odd count ends on one that computes nothing; the
-     * second half may have one block fewer) */
+     * last part may have fewer blocks) */
     for (int i = 0; i < L; i += 2) {
         PF2_STEP(i, st0, st1);
         PF2_STEP(i + 1, st1, st0);
     }
 #undef PF2_STEP
-    if constexpr (KS == 2) {
-        /* the second half's sums through LDS (its stage buffers are done) */
-        float* red = (float*)s_a[1];
-        if (kh == 1) {
+    if constexpr (KS > 1) {
+        /* the other parts' sums through LDS (the stages are done) */
+        float* red = (float*)s_a;
+        static_assert((KS - 1) * 32 * RW * TT * 4 <= (int)sizeof(s_a), "the sums fit the stages");
+        if (kh) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < NTL; t++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) red[(t * 16 + r) * (PF2_NT) + tid] = acc[t][r];
+                for (int r = 0; r < 16; r++) red[((kh - 1) * NTL * 16 + t * 16 + r) * NG + tid] = acc[t][r];
         }
         __syncthreads();
-        if (kh == 1) return;
+        if (kh) return;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int p = 0; p < KS - 1; p++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[t][r] = acc[t][r] + red[(t * 16 + r) * (PF2_NT) + tid];
+            for (int t = 0; t < NTL; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][r] = acc[t][r] + red[(p * NTL * 16 + t * 16 + r) * NG + tid];
     }
     if (row < R) {
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int tok = t0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -948,23 +962,56 @@ static bool pf_gemm16()
 
 bool lg_prefill_gemm16() { return pf_gemm16(); }
 
-/* the 32 x 32 product kernel (Q4_K, Q6_K): 128 rows x 64 tokens per
- * workgroup; two K halves in one workgroup where the tiles alone would give
- * one workgroup per CU or fewer (the 4096-row products at 512 tokens,
- * att_out and down: Q4_K 68.0 -> 61.8 us on average; Q|K|V's 384 tiles ran
- * faster unsplit, 48.7 against 55.2 us) */
+/* Tile (rows x tokens, K parts) of the 32 x 32 product kernels by the number
+ * of 32 x 32 output tiles.  A wave walks its part of K block by block, each
+ * waiting on loads that the block before issued, so its time is the number
+ * of blocks: where the wide tile would leave most of the 1024 SIMDs without
+ * a wave, smaller workgroups with K in more parts finish sooner, though they
+ * unpack each weight for fewer tokens.  Measured (us at the tile taken / at
+ * 128 x 64 with K in two parts, the former choice):
+ *   24576 x 4096, 512 tokens   Q4_K 170 / 178  (12288 tiles)
+ *    4096 x 4096, 512 tokens   Q4_K 27 (both)  (2048: a workgroup a CU, K in two)
+ *    4096 x 12288, 200 tokens  Q4_K 50 / 64, Q8_0 170 / 194, Q1_G 84 / 133  (896)
+ *    6144 x 4096, 77 tokens    Q4_K 20 / 24, Q1_G 30 / 47  (576)
+ *    4096 x 12288, 77 tokens   Q4_K 30 / 62, Q6_K 55 / 109, Q8_0 92 / 196  (384)
+ *    4096 x 12288, 16 tokens   Q4_K 21 / 60, Q6_K 35 / 109, Q1_G 35 / 130  (128)
+ *     600 x 2048, 96 tokens    Q4_K 6.7 / 14, Q6_K 9.3 / 22  (57)
+ * and on the other side of each line 24576 x 4096, 77 tokens (2304) Q4_K 45
+ * at 128 x 64, 48 at 64 x 32; 4096 x 4096, 200 tokens (896) Q4_K 20 with K
+ * in two parts, 24 in four. */
+enum { PF_T128x64, PF_T128x64_K2, PF_T64x32_K2, PF_T64x32_K4, PF_T32x32_K4 };
+static int pf_tile(int rows, int T)
+{
+    const long n32 = (long)((rows + 31) / 32) * ((T + 31) / 32);
+    if (n32 < 256) return PF_T32x32_K4;
+    if (n32 < 500) return PF_T64x32_K4;
+    if (n32 < 1800) return PF_T64x32_K2;
+    return (long)((rows + 127) / 128) * ((T + 63) / 64) <= 256 ? PF_T128x64_K2 : PF_T128x64;
+}
+
+template <int WT, int RW, int KS, int TT>
+static void k32_launch(const uint8_t* W, uint32_t rsz, int rows, int cols, const PfQ8K& x, int T, float* out, int ldo,
+                       int accumulate, hipStream_t s)
+{
+    const int nrb = ((rows + 32 * RW - 1) / (32 * RW) + 7) & ~7, ntl = (T + TT - 1) / TT;
+    const dim3 grid((unsigned)(nrb * ntl)), blk(64 * RW * KS);
+    if (accumulate) hipLaunchKernelGGL((k_pf_gemm_k32<WT, 1, RW, KS, TT>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo);
+    else hipLaunchKernelGGL((k_pf_gemm_k32<WT, 0, RW, KS, TT>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo);
+}
+
 template <int WT>
 static int gemm_k32(const uint8_t* W, uint32_t rsz, int rows, int cols, const PfQ8K& x, int T, float* out, int ldo,
                     int accumulate, hipStream_t s)
 {
-    const int nrb = (rows + PF2_RB - 1) / PF2_RB + 7 & ~7;
-    const int ntl = (T + 63) / 64;
-    const bool ks2 = nrb * ntl <= 256 && cols >= 4 * 256;
-    const dim3 grid((unsigned)(nrb * ntl)), blk(ks2 ? 2 * PF2_NT : PF2_NT);
-#define PF2_LAUNCH(A, N) hipLaunchKernelGGL((k_pf_gemm_k32<WT, A, N>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo)
-    if (accumulate) { if (ks2) PF2_LAUNCH(1, 2); else PF2_LAUNCH(1, 1); }
-    else { if (ks2) PF2_LAUNCH(0, 2); else PF2_LAUNCH(0, 1); }
-#undef PF2_LAUNCH
+#define K32(RW, KS, TT) k32_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
+    switch (pf_tile(rows, T)) {
+    case PF_T128x64: K32(4, 1, 64); break;
+    case PF_T128x64_K2: K32(4, 2, 64); break;
+    case PF_T64x32_K2: K32(2, 2, 32); break;
+    case PF_T64x32_K4: K32(2, 4, 32); break;
+    default: K32(1, 4, 32); break;
+    }
+#undef K32
     return lg_check_launch("prefill gemm");
 }
 
@@ -1635,11 +1682,9 @@ __global__ __launch_bounds__(512) void k_pf_gemm_b32(
     }
 }
 
-/* The same products on the 32 x 32 forms (k_pf_gemm_k32's tile: 128 rows
- * x 64 tokens per workgroup of 4 waves, a wave 32 rows x two 32-token C
- * tiles, the token tile of 8 blocks (256 values) a step staged two steps
- * ahead, K in two halves where the tiles alone would leave one workgroup
- * per CU).  Per 32-value block: the integer sum is one
+/* The same products on the 32 x 32 forms (k_pf_gemm_k32's tiles and parts of
+ * K, the token tile of 8 blocks (256 values) a step staged two steps ahead).
+ * Per 32-value block: the integer sum is one
  * v_mfma_i32_32x32x32_i8 (lane l: row l % 32's bytes 16 (l / 32) .. +15 of
  * the block -- Q8_0 quants, or Q1_0 bits as +-1 bytes -- against the
  * token's), and the scale d_w d_a of every (token, row) pair of the tile is
@@ -1656,56 +1701,59 @@ __global__ __launch_bounds__(512) void k_pf_gemm_b32(
  * dot_q8_0_q1_G's 2 s1 - asum, the scale MFMA puts d_a alone in place (B =
  * 1), and out += d_w sum_j d_a,j s_j per 128 values in k_pf_gemm_q1g's fp32
  * operations (the same bits where K is not split). */
-template <int WT, int ACC, int KS>
-__global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_gemm_b32x(
+template <int WT, int ACC, int RW, int KS, int TT>
+__global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2))) void k_pf_gemm_b32x(
     const uint8_t* __restrict__ W, uint32_t rsz, int R, int K, PfQ8K x, int T, float* __restrict__ out, int ldo)
 {
     constexpr bool G = WT == LG_Q1_G || WT == LG_Q1_G_R;   /* 128-value sign blocks */
     using B32 = PfB32<G ? LG_Q1_0 : WT>;
-    constexpr int TT = 64;
+    constexpr int NTL = TT / 32, NG = 64 * RW, NA = TT * 16 / NG, ND = TT * 8 / NG;
+    static_assert(NA * NG == TT * 16 && ND * NG == TT * 8, "stage pieces");
     __shared__ __attribute__((aligned(16))) int8_t s_a[KS][2][TT * PF2_AST];
     __shared__ __attribute__((aligned(16))) _Float16 s_d[KS][2][8][TT];   /* d_a per block of the step, per token */
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kh = wave >> 2, tid = threadIdx.x & (PF2_NT - 1);
+    const int kh = wave / RW, tid = threadIdx.x % NG;
     const int h = lane >> 5, j = lane & 31;
     const int nbk = K >> 5, nst = (nbk + 7) >> 3;
-    const int ns0 = KS == 2 ? (nst + 1) / 2 : nst;
-    const int s0 = kh * ns0, nsh = kh ? nst - ns0 : ns0, L = ns0;
+    const int L = (nst + KS - 1) / KS;
+    const int s0 = kh * L, nsh = min(L, nst - s0);   /* nsh may be <= 0 */
     const int nt = (T + TT - 1) / TT;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int rb = (slot / nt) * 8 + xcd;
-    if (rb * PF2_RB >= R) return;   /* padding of the row blocks to a multiple of 8 (whole workgroup) */
+    if (rb * 32 * RW >= R) return;   /* padding of the row blocks to a multiple of 8 (whole workgroup) */
     const int t0 = (slot % nt) * TT;
-    const int row = rb * PF2_RB + (wave & 3) * 32 + j;
+    const int row = (rb * RW + wave % RW) * 32 + j;
     const uint8_t* wr = W + (size_t)min(row, R - 1) * rsz;
     int8_t(*sa_)[TT * PF2_AST] = s_a[kh];
     _Float16(*sd_)[8][TT] = s_d[kh];
 
-    /* staging, per step: quant piece q = tid + 256 u (token q / 16, 16-byte
+    /* staging, per step: quant piece q = tid + NG u (token q / 16, 16-byte
      * piece q % 16 of the step's 256 values, clamped to the row's end), and
-     * d_a of blocks tid / 64 and tid / 64 + 4 of token tid % 64 */
+     * d_a of block q / TT of token q % TT */
     struct Stg {
-        v4i a[4];
-        float d[2];
+        v4i a[NA];
+        float d[ND];
     };
     auto stage_load = [&](Stg& st, int sp) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int q = tid + PF2_NT * u, tok = min(t0 + (q >> 4), T - 1);
+        for (int u = 0; u < NA; u++) {
+            const int q = tid + NG * u, tok = min(t0 + (q >> 4), T - 1);
             st.a[u] = *(const v4i*)(x.qs + (size_t)tok * K + min(sp * 256 + (q & 15) * 16, K - 16));
         }
-        const int tok = min(t0 + (tid & 63), T - 1);
 #pragma unroll
-        for (int e = 0; e < 2; e++) st.d[e] = x.d[(size_t)min(8 * sp + (tid >> 6) + 4 * e, nbk - 1) * x.tld + tok];
+        for (int e = 0; e < ND; e++) {
+            const int q = tid + NG * e;
+            st.d[e] = x.d[(size_t)min(8 * sp + q / TT, nbk - 1) * x.tld + min(t0 + q % TT, T - 1)];
+        }
     };
     auto stage_store = [&](const Stg& st, int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int q = tid + PF2_NT * u;
+        for (int u = 0; u < NA; u++) {
+            const int q = tid + NG * u;
             *(v4i*)(sa_[buf] + (q >> 4) * PF2_AST + (q & 15) * 16) = st.a[u];
         }
 #pragma unroll
-        for (int e = 0; e < 2; e++) sd_[buf][(tid >> 6) + 4 * e][tid & 63] = (_Float16)st.d[e];
+        for (int e = 0; e < ND; e++) sd_[buf][(tid + NG * e) / TT][(tid + NG * e) % TT] = (_Float16)st.d[e];
     };
     /* the lane's bytes of the step's 8 blocks and their d_w */
     struct Blk {
@@ -1759,9 +1807,9 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         }
     };
 
-    v16f acc[2];
-    acc[0] = (v16f){};
-    acc[1] = (v16f){};
+    v16f acc[NTL];
+#pragma unroll
+    for (int t = 0; t < NTL; t++) acc[t] = (v16f){};
 
     auto compute = [&](int buf, const Blk& cur, int sp) __attribute__((always_inline)) {
         const int8_t* sa = sa_[buf] + j * PF2_AST + 16 * h;
@@ -1774,7 +1822,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             for (int u = 0; u < 2; u++) {
                 const float dw = lg_h2f((uint16_t)cur.d[u]);
 #pragma unroll
-                for (int t = 0; t < 2; t++) {
+                for (int t = 0; t < NTL; t++) {
                     v16f g = (v16f){};
 #pragma unroll
                     for (int jj = 0; jj < 4; jj++) {
@@ -1804,7 +1852,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
             v8h bd = (v8h){};
             bd[0] = h ? (_Float16)0.0f : __builtin_bit_cast(_Float16, (uint16_t)(cur.d[e >> 1] >> (16 * (e & 1))));
 #pragma unroll
-            for (int t = 0; t < 2; t++) {
+            for (int t = 0; t < NTL; t++) {
                 const uint4 a = *(const uint4*)(sa + 32 * t * PF2_AST + 32 * e);
                 const v4i af = {(int)a.x, (int)a.y, (int)a.z, (int)a.w};
                 const v16i is = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, cur.q[e], (v16i){}, 0, 0, 0);
@@ -1818,7 +1866,7 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         }
     };
 
-    auto stp = [&](int i) { return s0 + min(i, nsh - 1); };
+    auto stp = [&](int i) { return min(s0 + max(min(i, nsh - 1), 0), nst - 1); };
     Blk cur, nxt;
     Stg st0, st1;
     stage_load(st0, stp(0));
@@ -1840,24 +1888,27 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
         PF3_STEP(i + 1, st1, st0);
     }
 #undef PF3_STEP
-    if constexpr (KS == 2) {
-        float* red = (float*)s_a[1];
-        if (kh == 1) {
+    if constexpr (KS > 1) {
+        float* red = (float*)s_a;
+        static_assert((KS - 1) * 32 * RW * TT * 4 <= (int)sizeof(s_a), "the sums fit the stages");
+        if (kh) {
 #pragma unroll
-            for (int t = 0; t < 2; t++)
+            for (int t = 0; t < NTL; t++)
 #pragma unroll
-                for (int r = 0; r < 16; r++) red[(t * 16 + r) * (PF2_NT) + tid] = acc[t][r];
+                for (int r = 0; r < 16; r++) red[((kh - 1) * NTL * 16 + t * 16 + r) * NG + tid] = acc[t][r];
         }
         __syncthreads();
-        if (kh == 1) return;
+        if (kh) return;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int p = 0; p < KS - 1; p++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[t][r] = acc[t][r] + red[(t * 16 + r) * (PF2_NT) + tid];
+            for (int t = 0; t < NTL; t++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[t][r] = acc[t][r] + red[(p * NTL * 16 + t * 16 + r) * NG + tid];
     }
     if (row < R) {
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
+        for (int t = 0; t < NTL; t++) {
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const int tok = t0 + 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
@@ -1870,18 +1921,29 @@ __global__ __launch_bounds__(PF2_NT * KS) __attribute__((amdgpu_waves_per_eu(2))
     }
 }
 
+template <int WT, int RW, int KS, int TT>
+static void b32x_launch(const uint8_t* W, uint32_t rsz, int rows, int cols, const PfQ8K& x, int T, float* out, int ldo,
+                        int accumulate, hipStream_t s)
+{
+    const int nrb = ((rows + 32 * RW - 1) / (32 * RW) + 7) & ~7, ntl = (T + TT - 1) / TT;
+    const dim3 grid((unsigned)(nrb * ntl)), blk(64 * RW * KS);
+    if (accumulate) hipLaunchKernelGGL((k_pf_gemm_b32x<WT, 1, RW, KS, TT>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo);
+    else hipLaunchKernelGGL((k_pf_gemm_b32x<WT, 0, RW, KS, TT>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo);
+}
+
 template <int WT>
 static int gemm_b32x(const uint8_t* W, uint32_t rsz, int rows, int cols, const PfQ8K& x, int T, float* out, int ldo,
                      int accumulate, hipStream_t s)
 {
-    const int nrb = (rows + PF2_RB - 1) / PF2_RB + 7 & ~7;
-    const int ntl = (T + 63) / 64;
-    const bool ks2 = nrb * ntl <= 256 && cols >= 4 * 256;
-    const dim3 grid((unsigned)(nrb * ntl)), blk(ks2 ? 2 * PF2_NT : PF2_NT);
-#define PF3_LAUNCH(A, N) hipLaunchKernelGGL((k_pf_gemm_b32x<WT, A, N>), grid, blk, 0, s, W, rsz, rows, cols, x, T, out, ldo)
-    if (accumulate) { if (ks2) PF3_LAUNCH(1, 2); else PF3_LAUNCH(1, 1); }
-    else { if (ks2) PF3_LAUNCH(0, 2); else PF3_LAUNCH(0, 1); }
-#undef PF3_LAUNCH
+#define B32X(RW, KS, TT) b32x_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
+    switch (pf_tile(rows, T)) {
+    case PF_T128x64: B32X(4, 1, 64); break;
+    case PF_T128x64_K2: B32X(4, 2, 64); break;
+    case PF_T64x32_K2: B32X(2, 2, 32); break;
+    case PF_T64x32_K4: B32X(2, 4, 32); break;
+    default: B32X(1, 4, 32); break;
+    }
+#undef B32X
     return lg_check_launch("prefill gemm (32-value blocks)");
 }
 

@@ -1,0 +1,43 @@
+"""The quantized token GEMMs (lg_matmul_tokens) at the edges of every tile the
+batched prefill picks -- 128 x 64, 64 x 32 and 32 x 32 with K in one, two or
+four parts, fewer blocks of K than parts, ends of rows and tokens -- against
+float64 over the same quantized operands."""
+import numpy as np
+import pytest
+import torch
+
+from ligguf_amd import encode, ops
+from ligguf_amd.lib import Q1_0, Q1_G, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, TYPE_NAMES, row_size
+
+pytestmark = pytest.mark.gpu
+
+# rows, width, tokens: 32 x 32 | 64 x 32, K in 4 | 64 x 32, K in 2 | 128 x 64, K in 2 | 128 x 64
+SHAPES = [(33, 256, 1), (600, 2304, 95), (4090, 1280, 33), (4097, 512, 65), (6145, 768, 100), (3970, 1280, 449), (12289, 512, 165)]
+TYPES = [Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, Q1_0, Q1_G]
+
+
+def activations(x, kq):
+    """float64 values of the rows of x as quantize_q8_K / quantize_q8_0 leave them"""
+    T, n = x.shape
+    raw = (ops.quantize_q8_K if kq else ops.quantize_q8_0)(x.reshape(-1)).cpu().numpy().reshape(T, -1)
+    size, d_bytes, count = (292, 4, 256) if kq else (34, 2, 32)
+    b = raw.reshape(T, n // count, size)
+    d = np.ascontiguousarray(b[:, :, :d_bytes]).view(np.float32 if kq else np.float16).astype(np.float64)
+    q = np.ascontiguousarray(b[:, :, d_bytes:d_bytes + count]).view(np.int8).astype(np.float64)
+    return torch.from_numpy((d * q).reshape(T, n)).to(x.device)
+
+
+@pytest.mark.parametrize("wt", TYPES, ids=[TYPE_NAMES[t] for t in TYPES])
+@pytest.mark.parametrize("R,n,T", SHAPES)
+def test_tiles(gpu, wt, R, n, T):
+    rsz = row_size(wt, n)
+    distinct = min(R, 512)   # encoding is host work: the rows repeat, with a stride that no tile edge divides
+    rows = encode.random_tensor(wt, R + n, wt, distinct, n).reshape(distinct, rsz)
+    rows = np.ascontiguousarray(rows[np.arange(R) * 37 % distinct])
+    w = torch.from_numpy(rows.reshape(-1)).to(gpu)
+    x = torch.from_numpy(np.random.default_rng(T).standard_normal((T, n)).astype(np.float32)).to(gpu)
+    wd = ops.dequantize_row(wt, w, R * n).reshape(R, n).double()
+    a = activations(x, wt not in (Q8_0, Q1_0, Q1_G))
+    got = ops.matmul_tokens(wt, w, rsz, n, R, x).double()
+    # the matvec bar: integer block sums are exact, their fp32 combination within 2e-6 of the sum of |terms|
+    assert bool(((got - a @ wd.T).abs() <= 2e-6 * (a.abs() @ wd.abs().T)).all())
