@@ -10,8 +10,11 @@
  * The reference runs the same arithmetic a token at a time through
  * matmul3/matmul (fast/lil_math.cpp:748-899); here each weight matrix is read
  * once per pass and multiplied on MFMA:
- *   - F32/F16 matrices x fp32 activations on v_mfma_f32_16x16x4f32: the
- *     products of dot_f32 / dot_f16_f32 exactly, fp32 accumulation;
+ *   - F32 matrices x fp32 activations on v_mfma_f32_16x16x4f32: the
+ *     products of dot_f32 exactly, fp32 accumulation;
+ *   - F16 matrices x fp32 activations, each in two fp16 parts, on fp16 MFMA
+ *     (lg_fgemm.hip): dot_f16_f32's products to 2^-21 of the activation; what
+ *     feeds them (LayerNorm, attention, GELU) writes the parts itself;
  *   - Q8_0/Q1_0/Q1_G matrices, repacked at upload into int8 values (the
  *     Q8_0 quants, or +-1 from the sign bits) and one fp32 scale per 32 --
  *     x Q8_0 activations (quantize_q8_0 per token, the same lane quantizer
@@ -50,7 +53,6 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 #define BERT_HD_MAX 128
 #define BERT_NCTX_MAX 4096
 #define BERT_NE_MAX 4096
-#define BERT_SP 16384          /* LDS floats for one attention block's scores */
 #define LG_VDB_KMAX 8
 #define VDB_BLOCKS_MAX 1024
 
@@ -90,7 +92,7 @@ template <int NP>
 __device__ __forceinline__ void b_layernorm(float (&v)[NP][4], int n, const float* __restrict__ w,
                                             const float* __restrict__ bias, float eps, double* red,
                                             float* __restrict__ out, int8_t* __restrict__ q, float* __restrict__ qd,
-                                            int ldd, int t)
+                                            int ldd, const HSplit& sp, int t)
 {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     double s = 0.0;
@@ -122,6 +124,7 @@ __device__ __forceinline__ void b_layernorm(float (&v)[NP][4], int n, const floa
                               : 0.0f;
         if (i0 < n) *(float4*)(out + i0) = make_float4(o[0], o[1], o[2], o[3]);
         if (q) b_emit_q8(o, q, qd, ldd, t, 4 * p + wv, n);
+        if (sp.h && i0 < n) lg_split_store4(o, 1.0f / sp.inv_all, sp, n, t, i0);
     }
 }
 
@@ -140,6 +143,7 @@ struct BEmbArgs {
     int8_t* q;                 /* optional Q8_0 of the output */
     float* qd;
     int ldd;
+    HSplit sp;                 /* optional split of the output (h NULL: none) */
 };
 
 template <int NP>
@@ -161,14 +165,14 @@ __global__ __launch_bounds__(256) void k_bert_embed(BEmbArgs a)
                               : 0.0f;
         }
     b_layernorm<NP>(v, a.n, a.w, a.b, a.eps, red, a.out + (size_t)t * a.n, a.q ? a.q + (size_t)t * a.n : nullptr, a.qd,
-                    a.ldd, t);
+                    a.ldd, a.sp, t);
 }
 
-/* LayerNorm of row t of y (n wide) into out, optionally quantized */
+/* LayerNorm of row t of y (n wide) into out, optionally quantized or split */
 template <int NP>
 __global__ __launch_bounds__(256) void k_bert_ln(const float* __restrict__ y, int n, const float* __restrict__ w,
                                                  const float* __restrict__ b, float eps, float* __restrict__ out,
-                                                 int8_t* __restrict__ q, float* __restrict__ qd, int ldd)
+                                                 int8_t* __restrict__ q, float* __restrict__ qd, int ldd, HSplit sp)
 {
     __shared__ double red[4];
     const int t = blockIdx.x;
@@ -181,7 +185,7 @@ __global__ __launch_bounds__(256) void k_bert_ln(const float* __restrict__ y, in
         const float4 x = i0 < n ? *(const float4*)(row + i0) : make_float4(0.f, 0.f, 0.f, 0.f);
         v[p][0] = x.x; v[p][1] = x.y; v[p][2] = x.z; v[p][3] = x.w;
     }
-    b_layernorm<NP>(v, n, w, b, eps, red, out + (size_t)t * n, q ? q + (size_t)t * n : nullptr, qd, ldd, t);
+    b_layernorm<NP>(v, n, w, b, eps, red, out + (size_t)t * n, q ? q + (size_t)t * n : nullptr, qd, ldd, sp, t);
 }
 
 /* Q8_0 of row t of x (n wide): the quantize_q8_0 matmul() applies before a
@@ -281,15 +285,15 @@ __global__ __launch_bounds__(64) void k_bert_gemm(BGemm a)
             }
         }
     } else {
-        constexpr int ESZ = WT == LG_F32 ? 4 : 2;
+        static_assert(WT == LG_F32, "F16 weights: lg_hgemm");
         const float* ap[TM];
         const uint8_t* bp[TN];
 #pragma unroll
         for (int i = 0; i < TM; i++) ap[i] = a.x + (size_t)tr[i] * a.ldx + 8 * g;
 #pragma unroll
-        for (int j = 0; j < TN; j++) bp[j] = a.w + ((size_t)wr[j] * a.K + 8 * g) * ESZ;
+        for (int j = 0; j < TN; j++) bp[j] = a.w + ((size_t)wr[j] * a.K + 8 * g) * 4;
         float4 A[NPF][TM][2];
-        uint4 B[NPF][TN][ESZ / 2];
+        uint4 B[NPF][TN][2];
         auto load = [&](int u, int k0) {
 #pragma unroll
             for (int i = 0; i < TM; i++) {
@@ -299,7 +303,7 @@ __global__ __launch_bounds__(64) void k_bert_gemm(BGemm a)
 #pragma unroll
             for (int j = 0; j < TN; j++)
 #pragma unroll
-                for (int h = 0; h < ESZ / 2; h++) B[u][j][h] = *(const uint4*)(bp[j] + (size_t)k0 * ESZ + 16 * h);
+                for (int h = 0; h < 2; h++) B[u][j][h] = *(const uint4*)(bp[j] + (size_t)k0 * 4 + 16 * h);
         };
         const int nc = a.K >> 5;
 #pragma unroll
@@ -319,21 +323,12 @@ __global__ __launch_bounds__(64) void k_bert_gemm(BGemm a)
                     }
 #pragma unroll
                     for (int j = 0; j < TN; j++) {
-                        if constexpr (WT == LG_F32) {
 #pragma unroll
-                            for (int h = 0; h < 2; h++) {
-                                bf[j][4 * h + 0] = __uint_as_float(B[u][j][h].x);
-                                bf[j][4 * h + 1] = __uint_as_float(B[u][j][h].y);
-                                bf[j][4 * h + 2] = __uint_as_float(B[u][j][h].z);
-                                bf[j][4 * h + 3] = __uint_as_float(B[u][j][h].w);
-                            }
-                        } else {
-                            const uint32_t uu[4] = {B[u][j][0].x, B[u][j][0].y, B[u][j][0].z, B[u][j][0].w};
-#pragma unroll
-                            for (int h = 0; h < 4; h++) {
-                                bf[j][2 * h] = lg_h2f((uint16_t)(uu[h] & 0xffffu));
-                                bf[j][2 * h + 1] = lg_h2f((uint16_t)(uu[h] >> 16));
-                            }
+                        for (int h = 0; h < 2; h++) {
+                            bf[j][4 * h + 0] = __uint_as_float(B[u][j][h].x);
+                            bf[j][4 * h + 1] = __uint_as_float(B[u][j][h].y);
+                            bf[j][4 * h + 2] = __uint_as_float(B[u][j][h].z);
+                            bf[j][4 * h + 3] = __uint_as_float(B[u][j][h].w);
                         }
                     }
 #pragma unroll
@@ -368,9 +363,7 @@ __global__ __launch_bounds__(64) void k_bert_gemm(BGemm a)
                 } else if constexpr (EP == EP_BIAS_RES) {
                     o = o + (bias + a.res[(size_t)t * a.ldr + r]);
                 } else {
-                    /* gelu (fast/lil_math.cpp:978-984) of row + bias */
-                    const float u = o + bias;
-                    o = 0.5f * u * (1.0f + tanhf(0.7978845608f * (u + 0.044715f * u * u * u)));
+                    o = lg_gelu(o + bias);
                 }
                 a.out[(size_t)t * a.ldo + r] = o;
             }
@@ -380,205 +373,181 @@ __global__ __launch_bounds__(64) void k_bert_gemm(BGemm a)
 /* ------------------------------------------------------------------ */
 /* bidirectional attention (fast/vdb.cpp:189-212)                       */
 /* ------------------------------------------------------------------ */
-/* One block per (block of qb query tokens of one sequence, head).  K and V
- * rows of the head stream through LDS in tiles of 64 positions; the qb
- * score rows (the whole sequence) stay in LDS: scores = q.k * scale, then
- * the reference's softmax (max, expf, sum, divide), then ctx = sum_t p_t v_t
- * in position order.  tpr = 256/qb threads share a query row. */
+/* One wave per (16 query tokens of one sequence, head), no LDS in the loop:
+ * S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x4f32, 32 keys a step,
+ * softmax online per query column in log2 units.
+ *
+ * The lane layouts need no shuffle between the two products.  A product's
+ * lane (g = l / 16, m = l % 16) holds A[m][k = g], B[k = g][m] and rows
+ * 4g..4g+3 of D's column m.  Which dimension of the head step j of S
+ * multiplies is free: lane group g takes its HD / 4 dimensions HD / 4 g + j,
+ * so a lane's K values are contiguous in the key's row.  D then holds keys
+ * 4g..4g+3 of query m, which are P^T's B operands when step v of the second
+ * product takes keys 4g + v; and with dimension NDT m + dt as row m of
+ * output tile dt, a lane's V values are contiguous too.  K and V come from
+ * L2 / L1 (16 rows of 128 bytes an instruction at HD = 32).
+ *
+ * What bounds it: latency; the MFMA needs 512 cycles per 16 x 16 tile at HD
+ * = 32 (4000 tokens of 64 to 190 positions: 7 of the 28 us a layer takes; K
+ * and V staged in LDS per 16 queries, the scores in LDS: 52).  Sequences up
+ * to ATT_ALONE positions: a workgroup's four waves take 16 queries each;
+ * longer ones: the four share 16 queries, wave w takes key steps w, w + 4,
+ * ..., the partial (max, sum, O) merged through LDS -- by the length alone,
+ * so that a text gives the same bits alone and in a batch. */
+#define ATT_ALONE 128
 struct BAttnBlk {
-    int q0, nq, s0, n;         /* first query token, queries, sequence start and length */
+    int q0, nq, s0, n;         /* first query token, queries (<= 64 / 16), sequence start and length */
 };
 
-template <int HD>
-__global__ __launch_bounds__(256) void k_bert_attn(const float* __restrict__ qkv, int ne,
-                                                   const BAttnBlk* __restrict__ blks, int qb, int pst, float scale,
-                                                   float* __restrict__ ctx)
+template <int N>
+__device__ __forceinline__ void b_ldn(float (&d)[N], const float* p)
 {
-    __shared__ float s_p[BERT_SP];
-    __shared__ float s_q[16][HD];
-    __shared__ float s_kv[64][HD + 1];
-    const BAttnBlk bk = blks[blockIdx.x];
-    const int h = blockIdx.y, tid = threadIdx.x;
-    const int tpr = 256 / qb;
-    const int qi = tid / tpr, kk = tid % tpr;
-    const size_t ld = 3 * (size_t)ne;
-    float* prow = s_p + qi * pst;
-
-    for (int idx = tid; idx < qb * HD; idx += 256) {
-        const int r = idx / HD, d = idx % HD;
-        s_q[r][d] = qkv[(size_t)(bk.q0 + min(r, bk.nq - 1)) * ld + h * HD + d];
-    }
-    for (int kt = 0; kt < bk.n; kt += 64) {
-        __syncthreads();
-        for (int idx = tid; idx < 64 * HD; idx += 256) {
-            const int r = idx / HD, d = idx % HD;
-            s_kv[r][d] = kt + r < bk.n ? qkv[(size_t)(bk.s0 + kt + r) * ld + ne + h * HD + d] : 0.0f;
-        }
-        __syncthreads();
-        for (int kj = kk; kj < 64; kj += tpr) {
-            float acc = 0.0f;
-#pragma unroll 16
-            for (int d = 0; d < HD; d++) acc = __builtin_fmaf(s_q[qi][d], s_kv[kj][d], acc);
-            if (kt + kj < bk.n) prow[kt + kj] = acc * scale;
-        }
-    }
-    __syncthreads();
-    /* softmax (fast/lil_math.cpp:964-976) over the row, tpr lanes per row */
-    float mx = -INFINITY;
-    for (int c = kk; c < bk.n; c += tpr) mx = fmaxf(mx, prow[c]);
-    for (int o = tpr >> 1; o; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    float sum = 0.0f;
-    for (int c = kk; c < bk.n; c += tpr) {
-        const float e = expf(prow[c] - mx);
-        prow[c] = e;
-        sum += e;
-    }
-    for (int o = tpr >> 1; o; o >>= 1) sum += __shfl_xor(sum, o);
-    for (int c = kk; c < bk.n; c += tpr) prow[c] = prow[c] / sum;
-
-    constexpr int DPT = HD / 16;
-    float acc[DPT];
+    if constexpr (N % 4 == 0) {
 #pragma unroll
-    for (int u = 0; u < DPT; u++) acc[u] = 0.0f;
-    for (int kt = 0; kt < bk.n; kt += 64) {
-        __syncthreads();
-        for (int idx = tid; idx < 64 * HD; idx += 256) {
-            const int r = idx / HD, d = idx % HD;
-            s_kv[r][d] = kt + r < bk.n ? qkv[(size_t)(bk.s0 + kt + r) * ld + 2 * ne + h * HD + d] : 0.0f;
+        for (int i = 0; i < N; i += 4) {
+            const float4 v = *(const float4*)(p + i);
+            d[i] = v.x; d[i + 1] = v.y; d[i + 2] = v.z; d[i + 3] = v.w;
         }
-        __syncthreads();
-        const int kn = min(64, bk.n - kt);
-        for (int kj = 0; kj < kn; kj++) {
-            const float p = prow[kt + kj];
+    } else if constexpr (N % 2 == 0) {
 #pragma unroll
-            for (int u = 0; u < DPT; u++) {
-                const int d = kk + tpr * u;
-                if (d < HD) acc[u] = __builtin_fmaf(p, s_kv[kj][d], acc[u]);
-            }
+        for (int i = 0; i < N; i += 2) {
+            const float2 v = *(const float2*)(p + i);
+            d[i] = v.x; d[i + 1] = v.y;
         }
-    }
-    if (qi < bk.nq) {
+    } else {
 #pragma unroll
-        for (int u = 0; u < DPT; u++) {
-            const int d = kk + tpr * u;
-            if (d < HD) ctx[(size_t)(bk.q0 + qi) * ne + h * HD + d] = acc[u];
-        }
+        for (int i = 0; i < N; i++) d[i] = p[i];
     }
 }
 
-/* The same on fp32 MFMA for sequences of up to PMAX positions: one block
- * per (16 query tokens of one sequence, head), 4 waves.  K, then V, come
- * into LDS in chunks of KC positions, each chunk with all its loads in
- * flight at once (the sequence is short: a handful of round trips in all).
- * Scores: wave w takes the 16-key tiles 16w, 16w+64, ... of a chunk; a
- * tile is S[q][key] = sum_d Q[q][d] K[key][d], HD/4 v_mfma_f32_16x16x4f32
- * (A = Q: lane (g, m) holds Q[m][d0+g]; B = K^T: K[key0+m][d0+g]; D:
- * queries 4g..4g+3, key m), scaled and kept in LDS.  The reference's
- * softmax runs on the rows as in k_bert_attn.  Then O[q][d] = sum_key
- * P[q][key] V[key][d]: per 4 keys one MFMA per 16 dims (A = P:
- * P[m][key0+g]; B = V: V[key0+g][16 dt + m]), wave w over the w-th quarter
- * of each chunk; the four waves' partial O are summed in LDS.  LDS rows are
- * padded to an odd number of floats so the 16 rows a lane group reads fall
- * in distinct banks. */
-template <int HD, int PMAX>
-struct BAttnChunk {
-    static constexpr int KC0 = HD <= 64 ? 256 : 128;
-    static constexpr int KC = KC0 < PMAX ? KC0 : PMAX;   /* positions per K/V chunk */
-};
-
-template <int HD, int PMAX>
-__global__ __launch_bounds__(256) void k_bert_attn_mfma(const float* __restrict__ qkv, int ne,
-                                                        const BAttnBlk* __restrict__ blks, float scale,
-                                                        float* __restrict__ ctx)
+template <int HD>
+__global__ __launch_bounds__(256) void k_bert_attn(const float* __restrict__ qkv, int ne, const BAttnBlk* __restrict__ blks,
+                                                   float scale, float* __restrict__ ctx, HSplit so)
 {
-    constexpr int LD = HD + 1, PS = PMAX + 1, NDT = HD / 16, KC = BAttnChunk<HD, PMAX>::KC, H4 = HD / 4;
-    __shared__ float s_q[16 * LD];
-    __shared__ float s_kv[KC * LD];
-    __shared__ float s_p[16 * PS];
-    const BAttnBlk bk = blks[blockIdx.x];
-    const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, m = lane & 15;
+    constexpr int NDT = HD / 16, DJ = HD / 4, KB = 32;
+    __shared__ float s_o[3 * 16 * HD];
+    __shared__ float s_ml[4 * 32];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, m = lane & 15, h = blockIdx.y;
+    BAttnBlk bk = blks[blockIdx.x];
+    const bool share = bk.n > ATT_ALONE;          /* workgroup-uniform */
+    const int ks = share ? wave : 0, kinc = share ? 4 * KB : KB;
+    if (!share) {
+        bk.q0 += 16 * wave;
+        bk.nq -= 16 * wave;
+        if (bk.nq <= 0) return;                   /* no barrier in this form */
+    }
     const size_t ld = 3 * (size_t)ne;
-
-    /* rows [c0, c0 + KC) of the head's K (off = ne) or V (off = 2 ne) into s_kv */
-    auto load_chunk = [&](int c0, int off) {
-        for (int idx = tid; idx < KC * H4; idx += 256) {
-            const int r = idx / H4, c4 = idx % H4;
-            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (c0 + r < bk.n) v = *(const float4*)(qkv + (size_t)(bk.s0 + c0 + r) * ld + off + h * HD + 4 * c4);
-            float* d = s_kv + r * LD + 4 * c4;
-            d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
-        }
-    };
-
-    for (int idx = tid; idx < 16 * HD; idx += 256) {
-        const int r = idx / HD, d = idx % HD;
-        s_q[r * LD + d] = qkv[(size_t)(bk.q0 + min(r, bk.nq - 1)) * ld + h * HD + d];
-    }
-    for (int c0 = 0; c0 < bk.n; c0 += KC) {
-        __syncthreads();
-        load_chunk(c0, ne);
-        __syncthreads();
-        const int kn = min(KC, bk.n - c0);
-        for (int k16 = 16 * w; k16 < kn; k16 += 64) {
-            v4f acc = (v4f){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int d0 = 0; d0 < HD; d0 += 4)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s_q[m * LD + d0 + g], s_kv[(k16 + m) * LD + d0 + g], acc, 0, 0,
-                                                           0);
-            const int key = c0 + k16 + m;
-            if (key < bk.n) {
-#pragma unroll
-                for (int v = 0; v < 4; v++) s_p[(4 * g + v) * PS + key] = acc[v] * scale;
-            }
-        }
-    }
-    __syncthreads();
-    {
-        /* softmax (fast/lil_math.cpp:964-976), 16 lanes per row */
-        const int qi = tid >> 4, kk = tid & 15;
-        float* prow = s_p + qi * PS;
-        float mx = -INFINITY;
-        for (int c = kk; c < bk.n; c += 16) mx = fmaxf(mx, prow[c]);
-#pragma unroll
-        for (int o = 8; o; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-        float sum = 0.0f;
-        for (int c = kk; c < bk.n; c += 16) {
-            const float e = expf(prow[c] - mx);
-            prow[c] = e;
-            sum += e;
-        }
-#pragma unroll
-        for (int o = 8; o; o >>= 1) sum += __shfl_xor(sum, o);
-        for (int c = kk; c < bk.n; c += 16) prow[c] = prow[c] / sum;
-    }
+    const float* kb = qkv + (size_t)bk.s0 * ld + ne + h * HD;
+    const float* vb = kb + ne;
+    float q[DJ];
+    b_ldn<DJ>(q, qkv + (size_t)(bk.q0 + min(m, bk.nq - 1)) * ld + h * HD + DJ * g);
     v4f o[NDT];
 #pragma unroll
     for (int dt = 0; dt < NDT; dt++) o[dt] = (v4f){0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < bk.n; c0 += KC) {
-        __syncthreads();
-        load_chunk(c0, 2 * ne);
-        __syncthreads();
-        const int kq = min(KC / 4, max(0, bk.n - c0 - w * (KC / 4)));   /* keys of this wave's quarter */
-        for (int k4 = 0; k4 < kq; k4 += 4) {
-            const int kl = w * (KC / 4) + k4;                            /* chunk-local key of the step */
-            const float pa = c0 + kl + g < bk.n ? s_p[m * PS + c0 + kl + g] : 0.0f;
+    float mx = -3.402823466e38f, sum = 0.0f;      /* finite: scores of -inf give p = 0, not NaN */
+
+    for (int k0 = KB * ks; k0 < bk.n; k0 += kinc) {
+        float kf[2][DJ], vf[2][4][NDT];
+#pragma unroll
+        for (int u = 0; u < 2; u++) b_ldn<DJ>(kf[u], kb + (size_t)min(k0 + 16 * u + m, bk.n - 1) * ld + DJ * g);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                b_ldn<NDT>(vf[u][v], vb + (size_t)min(k0 + 16 * u + 4 * g + v, bk.n - 1) * ld + NDT * m);
+        v4f st[2] = {(v4f){0.f, 0.f, 0.f, 0.f}, (v4f){0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int j = 0; j < DJ; j++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) st[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j], q[j], st[u], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 2; u++) st[u] *= scale;
+        if (k0 + KB > bk.n) {      /* keys past the end: p = 0, and 0 x V of the row that stands in must be 0 */
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    if (k0 + 16 * u + 4 * g + v >= bk.n) {
+                        st[u][v] = -INFINITY;
+#pragma unroll
+                        for (int dt = 0; dt < NDT; dt++) vf[u][v][dt] = 0.0f;
+                    }
+        }
+        float bm = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])),
+                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+        bm = fmaxf(bm, __shfl_xor(bm, 16));
+        bm = fmaxf(bm, __shfl_xor(bm, 32));
+        const float mn = fmaxf(mx, bm);
+        const float f = __builtin_amdgcn_exp2f((mx - mn) * 1.44269504f);
+        mx = mn;
+        float ps = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                st[u][v] = expf(st[u][v] - mn);
+                ps += st[u][v];
+            }
+        sum = __builtin_fmaf(sum, f, ps);      /* this lane's keys; the four groups meet at the end */
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) o[dt] *= f;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+#pragma unroll
+                for (int dt = 0; dt < NDT; dt++)
+                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][v][dt], st[u][v], o[dt], 0, 0, 0);
+    }
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    if (share) {
+        if (g == 0) {
+            s_ml[ks * 32 + m] = mx;
+            s_ml[ks * 32 + 16 + m] = sum;
+        }
+        if (ks)
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++)
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, s_kv[(kl + g) * LD + 16 * dt + m], o[dt], 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 4; v++) s_o[((ks - 1) * NDT * 4 + dt * 4 + v) * 64 + lane] = o[dt][v];
+        __syncthreads();
+        if (ks) return;
+        float mm = mx;
+#pragma unroll
+        for (int w = 1; w < 4; w++) mm = fmaxf(mm, s_ml[w * 32 + m]);
+        float f = __builtin_amdgcn_exp2f((mx - mm) * 1.44269504f);
+        sum *= f;
+#pragma unroll
+        for (int dt = 0; dt < NDT; dt++) o[dt] *= f;
+#pragma unroll
+        for (int w = 1; w < 4; w++) {
+            f = __builtin_amdgcn_exp2f((s_ml[w * 32 + m] - mm) * 1.44269504f);
+            sum = __builtin_fmaf(s_ml[w * 32 + 16 + m], f, sum);
+#pragma unroll
+            for (int dt = 0; dt < NDT; dt++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    o[dt][v] = __builtin_fmaf(s_o[((w - 1) * NDT * 4 + dt * 4 + v) * 64 + lane], f, o[dt][v]);
         }
     }
-    __syncthreads();
-    float* s_o = s_kv;                                   /* [4 waves][16 queries][HD] */
+    if (m >= bk.nq) return;
+    const int t = bk.q0 + m;
+    /* register v of tile dt is dimension NDT (4g + v) + dt: 4 NDT contiguous ones */
+    float r[4 * NDT];
 #pragma unroll
-    for (int dt = 0; dt < NDT; dt++)
+    for (int v = 0; v < 4; v++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) s_o[(w * 16 + 4 * g + v) * HD + 16 * dt + m] = o[dt][v];
-    __syncthreads();
-    for (int idx = tid; idx < 16 * HD; idx += 256) {
-        const int q = idx / HD, d = idx % HD;
-        if (q < bk.nq)
-            ctx[(size_t)(bk.q0 + q) * ne + h * HD + d] =
-                ((s_o[q * HD + d] + s_o[(16 + q) * HD + d]) + s_o[(32 + q) * HD + d]) + s_o[(48 + q) * HD + d];
+        for (int dt = 0; dt < NDT; dt++) r[v * NDT + dt] = o[dt][v] / sum;
+    const int i0 = h * HD + 4 * NDT * g;
+#pragma unroll
+    for (int i = 0; i < 4 * NDT; i += 4) {
+        if (so.h) {
+            const float v[4] = {r[i], r[i + 1], r[i + 2], r[i + 3]};
+            lg_split_store4(v, 1.0f / so.inv_all, so, ne, t, i0 + i);
+        } else {
+            *(float4*)(ctx + (size_t)t * ne + i0 + i) = make_float4(r[i], r[i + 1], r[i + 2], r[i + 3]);
+        }
     }
 }
 
@@ -629,6 +598,32 @@ __global__ __launch_bounds__(256) void k_bert_l2norm(float* __restrict__ emb, in
     if (ss <= 0.0f) return;
     const float inv = 1.0f / sqrtf(ss);
     for (int i = threadIdx.x; i < ne; i += 256) e[i] = e[i] * inv;
+}
+
+/* ------------------------------------------------------------------ */
+/* bounds of what an F16 matrix gives on LayerNorm output               */
+/* ------------------------------------------------------------------ */
+/* out = max over the rows (float bits) of a bound of |W_r . y + bias_r| for
+ * any LayerNorm output y = z lw + lb (|z|_2 <= sqrt(K)): sqrt(K) |W_r lw|_2 +
+ * sum |W_r lb| + |bias_r|.  One wave per row; *out starts at 0; a row that is
+ * not finite makes it infinite. */
+__global__ __launch_bounds__(256) void k_bert_bound(const uint16_t* __restrict__ W, int rows, int K,
+                                                    const float* __restrict__ lw, const float* __restrict__ lb,
+                                                    const float* __restrict__ bias, uint32_t* __restrict__ out)
+{
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (r >= rows) return;
+    float s2 = 0.0f, s1 = 0.0f;
+    for (int i = lane; i < K; i += 64) {
+        const float w = lg_h2f(W[(size_t)r * K + i]);
+        s2 = __builtin_fmaf(w * lw[i], w * lw[i], s2);
+        s1 += fabsf(w * lb[i]);
+    }
+    s2 = lg_group_sum<64>(s2);
+    s1 = lg_group_sum<64>(s1);
+    /* the sums' own rounding, and that of LayerNorm, is far inside the factor */
+    const float b = 1.001f * (sqrtf((float)K * s2) + s1 + fabsf(bias[r]));
+    if (lane == 0) atomicMax(out, b < INFINITY ? __float_as_uint(b) : 0x7f800000u);
 }
 
 /* ------------------------------------------------------------------ */
@@ -812,6 +807,9 @@ struct BLayer {
     BMat ao, up, down;
     float *ao_bias = nullptr, *up_bias = nullptr, *down_bias = nullptr;
     float *ln1_w = nullptr, *ln1_b = nullptr, *ln2_w = nullptr, *ln2_b = nullptr;
+    /* 2^-k of the split inputs of its F16 matrices, from bounds known at
+     * load: 0 where none is (the split then takes each token's own maximum) */
+    float in_inv = 0, ctx_inv = 0, x1_inv = 0, h_inv = 0;
 };
 
 struct lg_bert {
@@ -833,6 +831,8 @@ struct lg_bert {
     int8_t* aq = nullptr;
     float* ad = nullptr;
     int ldd = 0;
+    _Float16 *hx = nullptr, *hw = nullptr;   /* F16 matrices: split x / x1 and split ctx / h */
+    float* hinv = nullptr;                   /* [tmax] */
     /* per-pass tables: tokpos [tmax] int2, attention blocks, sequences */
     void* meta_dev = nullptr;
     uint8_t* meta_host = nullptr;   /* pinned */
@@ -996,6 +996,63 @@ static int bput_mat(lg_bert* b, const lg_weight* const* ws, int n, BMat& out)
     return LG_OK;
 }
 
+/* bound of |y_i| of a LayerNorm's output: |z_i| <= sqrt(n) */
+static float ln_bound(const float* w, const float* b, int n)
+{
+    float m = 0.0f;
+    for (int i = 0; i < n; i++) {
+        const float v = sqrtf((float)n) * fabsf(w[i]) + fabsf(b[i]);
+        m = v > m || v != v ? v : m;
+        if (m != m) return INFINITY;
+    }
+    return 1.001f * m;
+}
+
+/* 2^-k of a split whose values stay within bound; 0: no use as one */
+static float bound_inv(float bound) { return bound < 1e30f ? lg_pow2(-lg_split_exp(bound)) : 0.0f; }
+
+/* The scales of the split inputs of F16 matrices.  What feeds them is
+ * LayerNorm output, attention -- an average of V rows -- or GELU of an F16
+ * product of LayerNorm output: all bounded by the weights, so their producers
+ * write the split at once instead of a pass that looks for each token's
+ * largest value (k_hsplit).  A bound some 2^8 above the values a token shows
+ * leaves their parts 2^-31 of them apart. */
+static int bert_split_scales(lg_bert* b, const lg_bert_desc* m)
+{
+    const int ne = b->ne;
+    uint32_t* dev = nullptr;
+    int rc;
+    if ((rc = balloc(b, (void**)&dev, 8 * (size_t)b->n_layers))) return rc;
+    std::vector<uint32_t> hb(2 * (size_t)b->n_layers, 0u);
+    if (b->n_layers) LG_HIP_CHECK(hipMemcpy(dev, hb.data(), hb.size() * 4, hipMemcpyHostToDevice));
+    auto bound = [&](const BMat& W, int row0, const float* lw, const float* lb, const float* bias, uint32_t* out) {
+        const int rows = W.rows - row0;
+        hipLaunchKernelGGL(k_bert_bound, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, b->stream,
+                           (const uint16_t*)W.w + (size_t)row0 * W.cols, rows, W.cols, lw, lb, bias, out);
+    };
+    for (int l = 0; l < b->n_layers; l++) {
+        const BLayer& L = b->layers[l];
+        const float* lw = l ? b->layers[l - 1].ln2_w : b->emb_w;
+        const float* lb = l ? b->layers[l - 1].ln2_b : b->emb_b;
+        const BMat& v = L.qkv[L.nqkv - 1];
+        if (v.type == LG_F16) bound(v, L.nqkv == 1 ? 2 * ne : 0, lw, lb, L.qkv_bias + 2 * ne, dev + 2 * l);
+        if (L.up.type == LG_F16) bound(L.up, 0, L.ln1_w, L.ln1_b, L.up_bias, dev + 2 * l + 1);
+    }
+    if ((rc = lg_check_launch("bert bounds"))) return rc;
+    LG_HIP_CHECK(hipStreamSynchronize(b->stream));
+    if (b->n_layers) LG_HIP_CHECK(hipMemcpy(hb.data(), dev, hb.size() * 4, hipMemcpyDeviceToHost));
+    for (int l = 0; l < b->n_layers; l++) {
+        BLayer& L = b->layers[l];
+        L.in_inv = bound_inv(l ? ln_bound(m->layers[l - 1].ffn_norm_w, m->layers[l - 1].ffn_norm_b, ne)
+                               : ln_bound(m->emb_norm_w, m->emb_norm_b, ne));
+        L.x1_inv = bound_inv(ln_bound(m->layers[l].attn_norm_w, m->layers[l].attn_norm_b, ne));
+        const uint32_t* u = hb.data() + 2 * l;
+        if (L.qkv[L.nqkv - 1].type == LG_F16) L.ctx_inv = bound_inv(__builtin_bit_cast(float, u[0]));
+        if (L.up.type == LG_F16) L.h_inv = bound_inv(__builtin_bit_cast(float, u[1]));
+    }
+    return LG_OK;
+}
+
 static int bert_load_impl(lg_bert* b, const lg_bert_desc* m, int max_tokens)
 {
     const int ne = m->n_embed, nff = m->n_ff;
@@ -1078,6 +1135,8 @@ static int bert_load_impl(lg_bert* b, const lg_bert_desc* m, int max_tokens)
             return rc;
     }
 
+    if ((rc = bert_split_scales(b, m))) return rc;
+
     /* activations for tmax tokens */
     int tmax = max_tokens > 0 ? max_tokens : std::max(m->n_context, 4096);
     if (tmax < m->n_context) { lg_set_error("bert load: max_tokens %d below n_context %d", tmax, m->n_context); return LG_ERR_ARG; }
@@ -1089,6 +1148,9 @@ static int bert_load_impl(lg_bert* b, const lg_bert_desc* m, int max_tokens)
         (rc = balloc(b, (void**)&b->y, T * ne * 4)) || (rc = balloc(b, (void**)&b->qkv, T * 3 * ne * 4)) ||
         (rc = balloc(b, (void**)&b->ctx, T * ne * 4)) || (rc = balloc(b, (void**)&b->h, T * nff * 4)) ||
         (rc = balloc(b, (void**)&b->aq, T * wmax)) || (rc = balloc(b, (void**)&b->ad, T * (wmax / 32) * 4)) ||
+        (rc = balloc(b, (void**)&b->hx, lg_hsplit_bytes((int)T, ne))) ||
+        (rc = balloc(b, (void**)&b->hw, lg_hsplit_bytes((int)T, (int)wmax))) ||
+        (rc = balloc(b, (void**)&b->hinv, T * 4)) ||
         (rc = balloc(b, (void**)&b->emb_dev, (T / 2) * ne * 4)) || (rc = balloc(b, (void**)&b->q_emb_dev, (size_t)ne * 4)))
         return rc;
     /* tables: tokpos T int2, attention blocks (<= T/4 + T/2) x 4 ints, sequences T/2 int2 */
@@ -1133,18 +1195,27 @@ static void gemm_tiles(const BGemm& a, hipStream_t s)
     else gemm_launch<WT, EP, 1, 1>(a, s);
 }
 
+/* xs: the split of x, which F16 matrices read (h NULL: taken here from x
+ * into hw, each token's own scale); so: where EP_BIAS_GELU_SPLIT writes */
 template <int EP>
-static int gemm_ep(const BMat& W, const float* x, int ldx, const lg_bert* b, int T, const float* bias, const float* res,
-                   int ldr, float* out, int ldo)
+static int gemm_ep(const BMat& W, const float* x, int ldx, HSplit xs, const lg_bert* b, int T, const float* bias,
+                   const float* res, int ldr, float* out, int ldo, HSplit so = HSplit{})
 {
     BGemm a;
     a.w = W.w; a.wd = W.d; a.R = W.rows; a.K = W.cols;
     a.x = x; a.ldx = ldx; a.q = b->aq; a.qd = b->ad; a.ldd = b->ldd;
-    a.T = T; a.bias = bias; a.res = res; a.ldr = ldr; a.out = out; a.ldo = ldo;
-    switch (W.type) {
-    case LG_F32: gemm_tiles<LG_F32, EP>(a, b->stream); break;
-    case LG_F16: gemm_tiles<LG_F16, EP>(a, b->stream); break;
-    default: gemm_tiles<BF_I8, EP>(a, b->stream); break;
+    a.T = T; a.bias = bias; a.res = res; a.ldr = ldr; a.out = out; a.ldo = ldo; a.so = so;
+    if (W.type == LG_F16) {
+        if (!xs.h) {
+            xs = HSplit{b->hw, b->hinv, 0.0f};
+            const int rc = lg_hsplit(x, ldx, W.cols, T, xs, b->stream);
+            if (rc) return rc;
+        }
+        return lg_hgemm(a, xs, EP, b->stream);
+    }
+    if constexpr (EP != EP_BIAS_GELU_SPLIT) {
+        if (W.type == LG_F32) gemm_tiles<LG_F32, EP>(a, b->stream);
+        else gemm_tiles<BF_I8, EP>(a, b->stream);
     }
     return lg_check_launch("bert gemm");
 }
@@ -1171,12 +1242,13 @@ static int launch_quant(const lg_bert* b, const float* x, int n, int T)
     return lg_check_launch("bert quant");
 }
 
-static int launch_ln(const lg_bert* b, const float* y, const float* w, const float* bias, float* out, bool quant, int T)
+static int launch_ln(const lg_bert* b, const float* y, const float* w, const float* bias, float* out, bool quant, const HSplit& sp,
+                     int T)
 {
     const int np = (b->ne + 1023) / 1024;
     int8_t* q = quant ? b->aq : nullptr;
 #define LN_CASE(NP) \
-    case NP: hipLaunchKernelGGL(k_bert_ln<NP>, dim3(T), dim3(256), 0, b->stream, y, b->ne, w, bias, b->eps, out, q, b->ad, b->ldd); break
+    case NP: hipLaunchKernelGGL(k_bert_ln<NP>, dim3(T), dim3(256), 0, b->stream, y, b->ne, w, bias, b->eps, out, q, b->ad, b->ldd, sp); break
     switch (np) {
         LN_CASE(1); LN_CASE(2); LN_CASE(3); LN_CASE(4);
     default: lg_set_error("bert: n_embed %d", b->ne); return LG_ERR_ARG;
@@ -1203,15 +1275,26 @@ static int trace_copy(const lg_bert* b, int l, int s, int K, int T)
     return LG_OK;
 }
 
-static bool any_i8(const BLayer& L)
+static bool any_of(const BLayer& L, int type)
 {
     for (int i = 0; i < L.nqkv; i++)
-        if (L.qkv[i].type == BF_I8) return true;
+        if (L.qkv[i].type == type) return true;
     return false;
+}
+static bool any_i8(const BLayer& L) { return any_of(L, BF_I8); }
+
+/* the split that a producer writes for F16 consumers (h NULL: none) */
+static HSplit split_for(bool wanted, _Float16* h, float inv) { return wanted && inv > 0.0f ? HSplit{h, nullptr, inv} : HSplit{}; }
+
+/* x's split for layer l's Q|K|V */
+static HSplit x_split(const lg_bert* b, int l)
+{
+    if (l >= b->n_layers) return HSplit{};
+    return split_for(any_of(b->layers[l], LG_F16), b->hx, b->layers[l].in_inv);
 }
 
 /* the encoder over the T tokens whose tables are in meta_dev */
-static int bert_layers(lg_bert* b, int T, int nblk, int qb, int pst, int nseq)
+static int bert_layers(lg_bert* b, int T, int nblk, int nseq)
 {
     const int ne = b->ne;
     const int2* tokpos = (const int2*)b->meta_dev;
@@ -1226,6 +1309,7 @@ static int bert_layers(lg_bert* b, int T, int nblk, int qb, int pst, int nseq)
         a.tokpos = tokpos; a.w = b->emb_w; a.b = b->emb_b; a.eps = b->eps; a.n = ne; a.out = b->x;
         a.q = (b->n_layers > 0 && any_i8(b->layers[0])) ? b->aq : nullptr;
         a.qd = b->ad; a.ldd = b->ldd;
+        a.sp = x_split(b, 0);
         switch ((ne + 1023) / 1024) {
         case 1: hipLaunchKernelGGL(k_bert_embed<1>, dim3(T), dim3(256), 0, b->stream, a); break;
         case 2: hipLaunchKernelGGL(k_bert_embed<2>, dim3(T), dim3(256), 0, b->stream, a); break;
@@ -1238,30 +1322,25 @@ static int bert_layers(lg_bert* b, int T, int nblk, int qb, int pst, int nseq)
     const float scale = 1.0f / sqrtf((float)b->hd);
     for (int l = 0; l < b->n_layers; l++) {
         const BLayer& L = b->layers[l];
+        const HSplit xs = x_split(b, l);
+        const HSplit cs = split_for(L.ao.type == LG_F16, b->hw, L.ctx_inv);
+        const HSplit x1s = split_for(L.up.type == LG_F16, b->hx, L.x1_inv);
+        /* (up's own input would be split into hw where x1s is none) */
+        const HSplit hs = split_for(L.down.type == LG_F16 && x1s.h, b->hw, L.h_inv);
         /* q|k|v = W x + bias (fast/vdb.cpp:180-186) */
         if (L.nqkv == 1) {
-            if ((rc = gemm_ep<EP_BIAS>(L.qkv[0], b->x, ne, b, T, L.qkv_bias, nullptr, 0, b->qkv, 3 * ne))) return rc;
+            if ((rc = gemm_ep<EP_BIAS>(L.qkv[0], b->x, ne, xs, b, T, L.qkv_bias, nullptr, 0, b->qkv, 3 * ne))) return rc;
         } else {
             /* mixed forms: x's Q8_0 (if any of them needs it) came with x */
             for (int i = 0; i < 3; i++)
-                if ((rc = gemm_ep<EP_BIAS>(L.qkv[i], b->x, ne, b, T, L.qkv_bias + i * ne, nullptr, 0, b->qkv + i * ne, 3 * ne)))
+                if ((rc = gemm_ep<EP_BIAS>(L.qkv[i], b->x, ne, xs, b, T, L.qkv_bias + i * ne, nullptr, 0, b->qkv + i * ne,
+                                           3 * ne)))
                     return rc;
         }
         /* attention (fast/vdb.cpp:189-212) */
         const dim3 ag((unsigned)nblk, (unsigned)b->nh);
-#define ATT_CASE(HD)                                                                                                  \
-    case HD:                                                                                                          \
-        if (pst <= 128)                                                                                               \
-            hipLaunchKernelGGL((k_bert_attn_mfma<HD, 128>), ag, dim3(256), 0, b->stream, b->qkv, ne, blks, scale, b->ctx); \
-        else if (pst <= 256)                                                                                          \
-            hipLaunchKernelGGL((k_bert_attn_mfma<HD, 256>), ag, dim3(256), 0, b->stream, b->qkv, ne, blks, scale, b->ctx); \
-        else if (pst <= 512)                                                                                          \
-            hipLaunchKernelGGL((k_bert_attn_mfma<HD, 512>), ag, dim3(256), 0, b->stream, b->qkv, ne, blks, scale, b->ctx); \
-        else if (pst <= 1024)                                                                                         \
-            hipLaunchKernelGGL((k_bert_attn_mfma<HD, 1024>), ag, dim3(256), 0, b->stream, b->qkv, ne, blks, scale, b->ctx); \
-        else                                                                                                          \
-            hipLaunchKernelGGL(k_bert_attn<HD>, ag, dim3(256), 0, b->stream, b->qkv, ne, blks, qb, pst, scale, b->ctx); \
-        break
+#define ATT_CASE(HD) \
+    case HD: hipLaunchKernelGGL(k_bert_attn<HD>, ag, dim3(256), 0, b->stream, b->qkv, ne, blks, scale, b->ctx, cs); break
         switch (b->hd) {
             ATT_CASE(16); ATT_CASE(32); ATT_CASE(48); ATT_CASE(64); ATT_CASE(80); ATT_CASE(96); ATT_CASE(112); ATT_CASE(128);
         default: lg_set_error("bert: head_dim %d", b->hd); return LG_ERR_ARG;
@@ -1270,16 +1349,18 @@ static int bert_layers(lg_bert* b, int T, int nblk, int qb, int pst, int nseq)
         if ((rc = lg_check_launch("bert attention"))) return rc;
         /* x1 = layernorm(att_out ctx + bias + x) (fast/vdb.cpp:219-222) */
         if (L.ao.type == BF_I8 && ((rc = launch_quant(b, b->ctx, ne, T)) || (rc = trace_copy(b, l, 1, ne, T)))) return rc;
-        if ((rc = gemm_ep<EP_BIAS_RES>(L.ao, b->ctx, ne, b, T, L.ao_bias, b->x, ne, b->y, ne))) return rc;
-        if ((rc = launch_ln(b, b->y, L.ln1_w, L.ln1_b, b->x1, L.up.type == BF_I8, T))) return rc;
+        if ((rc = gemm_ep<EP_BIAS_RES>(L.ao, b->ctx, ne, cs, b, T, L.ao_bias, b->x, ne, b->y, ne))) return rc;
+        if ((rc = launch_ln(b, b->y, L.ln1_w, L.ln1_b, b->x1, L.up.type == BF_I8, x1s, T))) return rc;
         if (L.up.type == BF_I8 && (rc = trace_copy(b, l, 2, ne, T))) return rc;
         /* h = gelu(up x1 + bias); x = layernorm(down h + bias + x1) (:224-231) */
-        if ((rc = gemm_ep<EP_BIAS_GELU>(L.up, b->x1, ne, b, T, L.up_bias, nullptr, 0, b->h, b->nff))) return rc;
+        if (hs.h) rc = gemm_ep<EP_BIAS_GELU_SPLIT>(L.up, b->x1, ne, x1s, b, T, L.up_bias, nullptr, 0, nullptr, 0, hs);
+        else rc = gemm_ep<EP_BIAS_GELU>(L.up, b->x1, ne, x1s, b, T, L.up_bias, nullptr, 0, b->h, b->nff);
+        if (rc) return rc;
         if (L.down.type == BF_I8 && ((rc = launch_quant(b, b->h, b->nff, T)) || (rc = trace_copy(b, l, 3, b->nff, T))))
             return rc;
-        if ((rc = gemm_ep<EP_BIAS_RES>(L.down, b->h, b->nff, b, T, L.down_bias, b->x1, ne, b->y, ne))) return rc;
+        if ((rc = gemm_ep<EP_BIAS_RES>(L.down, b->h, b->nff, hs, b, T, L.down_bias, b->x1, ne, b->y, ne))) return rc;
         const bool qn = l + 1 < b->n_layers && any_i8(b->layers[l + 1]);
-        if ((rc = launch_ln(b, b->y, L.ln2_w, L.ln2_b, b->x, qn, T))) return rc;
+        if ((rc = launch_ln(b, b->y, L.ln2_w, L.ln2_b, b->x, qn, x_split(b, l + 1), T))) return rc;
         if (qn && (rc = trace_copy(b, l + 1, 0, ne, T))) return rc;
     }
     hipLaunchKernelGGL(k_bert_pool_mean, dim3(nseq, (ne + 63) / 64), dim3(1024), 0, b->stream, b->x, ne, seqs,
@@ -1289,9 +1370,6 @@ static int bert_layers(lg_bert* b, int T, int nblk, int qb, int pst, int nseq)
     return lg_check_launch("bert l2norm");
 }
 
-/* the attention query block for the longest sequence of a pass */
-static int attn_qb(int nmax) { return nmax <= 1024 ? 16 : nmax <= 2048 ? 8 : 4; }
-
 /* Embed sequences [s_begin, s_end) of (toks, offsets) in one pass; the
  * caller has checked that their wrapped lengths fit tmax. */
 static int bert_pass(lg_bert* b, const int* toks, const int* offsets, int s_begin, int s_end, float* out_host)
@@ -1300,10 +1378,6 @@ static int bert_pass(lg_bert* b, const int* toks, const int* offsets, int s_begi
     int2* tokpos = (int2*)b->meta_host;
     BAttnBlk* blks = (BAttnBlk*)(b->meta_host + (size_t)b->tmax * 8);
     int2* seqs = (int2*)((uint8_t*)blks + ((size_t)b->tmax / 4 + b->tmax / 2 + 1) * sizeof(BAttnBlk));
-    int nmax = 0;
-    for (int s = s_begin; s < s_end; s++) nmax = std::max(nmax, std::min(offsets[s + 1] - offsets[s], b->nctx - 2) + 2);
-    const int qb = attn_qb(nmax);
-    const int pst = (nmax + 63) & ~63;
     int T = 0, nblk = 0;
     for (int s = s_begin; s < s_end; s++) {
         const int raw = std::min(offsets[s + 1] - offsets[s], b->nctx - 2);   /* toks.resize(n_context - 2) */
@@ -1311,6 +1385,7 @@ static int bert_pass(lg_bert* b, const int* toks, const int* offsets, int s_begi
         tokpos[T] = make_int2(b->tok_cls, 0);
         for (int i = 0; i < raw; i++) tokpos[T + 1 + i] = make_int2(toks[offsets[s] + i], 1 + i);
         tokpos[T + n - 1] = make_int2(b->tok_sep, n - 1);
+        const int qb = n > ATT_ALONE ? 16 : 64;
         for (int q = 0; q < n; q += qb) blks[nblk++] = BAttnBlk{T + q, std::min(qb, n - q), T, n};
         seqs[s - s_begin] = make_int2(T, n);
         T += n;
@@ -1321,7 +1396,7 @@ static int bert_pass(lg_bert* b, const int* toks, const int* offsets, int s_begi
             return LG_ERR_ARG;
         }
     LG_HIP_CHECK(hipMemcpyAsync(b->meta_dev, b->meta_host, b->meta_bytes, hipMemcpyHostToDevice, b->stream));
-    int rc = bert_layers(b, T, nblk, qb, pst, nseq);
+    int rc = bert_layers(b, T, nblk, nseq);
     b->trace = nullptr;                                  /* one pass only */
     if (rc) return rc;
     if (out_host) {

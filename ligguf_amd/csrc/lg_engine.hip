@@ -1615,7 +1615,7 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
     q.d = (float*)(ws + o_d);
     q.bs = (int16_t*)(ws + o_bs);
     q.as = (int*)(ws + o_as);
-    if (at == LG_F16) q.hs = HSplit{(_Float16*)ws, (float*)(ws + o_inv)};
+    if (at == LG_F16) q.hs = HSplit{(_Float16*)ws, (float*)(ws + o_inv), 0.0f};
     int rc = lg_prefill_quantize(at, x, n, nullptr, 0.0f, n, T, q, (hipStream_t)stream);
     if (!rc) rc = lg_prefill_gemm(type, (const uint8_t*)w, rsz, d, n, q, T, out, d, 0, (hipStream_t)stream);
     const hipError_t e2 = hipStreamSynchronize((hipStream_t)stream);

@@ -5,8 +5,20 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
-/* epilogues; STORE / ADD: no bias; ADD: out += */
-enum { EP_BIAS = 0, EP_BIAS_RES = 1, EP_BIAS_GELU = 2, EP_STORE = 3, EP_ADD = 4 };
+/* epilogues; STORE / ADD: no bias; ADD: out +=; BIAS_GELU_SPLIT: BIAS_GELU
+ * with its values split for the next F16 GEMM (lg_hgemm only) */
+enum { EP_BIAS = 0, EP_BIAS_RES = 1, EP_BIAS_GELU = 2, EP_BIAS_GELU_SPLIT = 3, EP_STORE = 4, EP_ADD = 5 };
+
+/* Split activations of T tokens of K values (a multiple of 32): each fp32
+ * value times its token's power of two 1 / inv[t] as fp16 hi (rounded toward
+ * zero) and lo = fp16 of the rest, laid out [t][K / 32][hi 32 | lo 32].  The
+ * power puts the token's largest finite |x|, or a bound of it, in [2^14,
+ * 2^15).  inv NULL: every token's is inv_all. */
+struct HSplit {
+    _Float16* h;
+    float* inv;
+    float inv_all;
+};
 
 struct BGemm {
     const uint8_t* w;          /* F32/F16: [R][K]; BF_I8: int8 [R][K] */
@@ -23,15 +35,7 @@ struct BGemm {
     int ldr;
     float* out;                /* [T][ldo] */
     int ldo;
-};
-
-/* Split activations of T tokens of K values (a multiple of 32): each fp32
- * value times its token's power of two 1 / inv[t] -- the token's largest
- * finite |x| lands in [2^14, 2^15) -- as fp16 hi (rounded toward zero) and
- * lo = fp16 of the rest, laid out [t][K / 32][hi 32 | lo 32]. */
-struct HSplit {
-    _Float16* h;
-    float* inv;
+    HSplit so;                 /* EP_BIAS_GELU_SPLIT: the output, R values a token (a multiple of 32), inv_all a power of two */
 };
 
 /* bytes of h for T tokens of K values (as many as the fp32 rows) */
@@ -44,16 +48,16 @@ int lg_hsplit(const float* x, int ldx, int K, int T, const HSplit& o, hipStream_
 int lg_hgemm(const BGemm& a, const HSplit& x, int ep, hipStream_t s);
 
 #ifdef __HIPCC__
-/* ---- device side of the split, for the kernels that produce activations ---- */
-
-/* k of the token's scale 2^k from the largest finite |x| (0: any) */
-__device__ __forceinline__ int lg_split_exp(float amax)
+/* k of a token's scale 2^k from its largest finite |x| (0: any) */
+__host__ __device__ __forceinline__ int lg_split_exp(float amax)
 {
-    const int k = 141 - (int)(__float_as_uint(amax) >> 23);   /* amax 2^k in [2^14, 2^15) */
-    return k > 126 ? 126 : k;                                  /* both 2^k and 2^-k normal */
+    const int k = 141 - (int)(__builtin_bit_cast(uint32_t, amax) >> 23);   /* amax 2^k in [2^14, 2^15) */
+    return k > 126 ? 126 : k;                                               /* both 2^k and 2^-k normal */
 }
 
-__device__ __forceinline__ float lg_pow2(int k) { return __uint_as_float((uint32_t)(127 + k) << 23); }
+__host__ __device__ __forceinline__ float lg_pow2(int k) { return __builtin_bit_cast(float, (uint32_t)(127 + k) << 23); }
+
+/* ---- device side of the split, for the kernels that produce activations ---- */
 
 /* |x| for the maximum: infinities and NaN take no part */
 __device__ __forceinline__ float lg_finite_abs(float x)
@@ -83,6 +87,20 @@ __device__ __forceinline__ void lg_split2(float x0, float x1, float s, uint32_t&
     const uint32_t hb = __builtin_bit_cast(uint32_t, h), lb = __builtin_bit_cast(uint32_t, l);
     hi = lg_nonzero_half(hb & 0xffffu, v0) | (lg_nonzero_half(hb >> 16, v1) << 16);
     lo = lg_nonzero_half(lb & 0xffffu, v0) | (lg_nonzero_half(lb >> 16, v1) << 16);
+}
+
+/* one value: hi in the low half, lo in the high half */
+__device__ __forceinline__ uint32_t lg_split1(float x, float s)
+{
+    uint32_t hi, lo;
+    lg_split2(x, 0.0f, s, hi, lo);
+    return (hi & 0xffffu) | (lo << 16);
+}
+
+/* gelu (fast/lil_math.cpp:978-984) */
+__device__ __forceinline__ float lg_gelu(float g)
+{
+    return 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));
 }
 
 /* four values i .. i + 3 (i a multiple of 4) of token t into the split rows */

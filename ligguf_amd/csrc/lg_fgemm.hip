@@ -49,6 +49,31 @@ int lg_hsplit(const float* x, int ldx, int K, int T, const HSplit& o, hipStream_
     return lg_check_launch("activation split");
 }
 
+/* one output: the sum `acc` of token t (t >= T: not stored) and weight row
+ * `row`; the lanes of a 32-lane half hold consecutive rows */
+template <int EP>
+__device__ __forceinline__ void hg_emit(const BGemm& a, float acc, float inv, float bias, int t, int row)
+{
+    const float o = acc * inv;
+    if constexpr (EP == EP_BIAS_GELU_SPLIT) {
+        /* a lane and its neighbour hold two rows of a token: the even one
+         * stores both high parts, the odd one both low ones */
+        const uint32_t w = lg_split1(lg_gelu(o + bias), 1.0f / a.so.inv_all);
+        const uint32_t n = (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xb1, 0xf, 0xf, true);   /* lane ^ 1 */
+        const int odd = row & 1;
+        uint32_t* p = (uint32_t*)(a.so.h + (size_t)(row >> 5) * 64 + (row & 30) + 32 * odd);
+        if (t < a.T) p[(size_t)t * a.R] = odd ? (n >> 16) | (w & 0xffff0000u) : (w & 0xffffu) | (n << 16);
+        return;
+    }
+    if (t >= a.T) return;
+    float* p = a.out + (size_t)t * a.ldo + row;
+    if constexpr (EP == EP_STORE) *p = o;
+    else if constexpr (EP == EP_ADD) *p = *p + o;
+    else if constexpr (EP == EP_BIAS) *p = o + bias;
+    else if constexpr (EP == EP_BIAS_RES) *p = o + (bias + a.res[(size_t)t * a.ldr + row]);
+    else *p = lg_gelu(o + bias);
+}
+
 /* A workgroup computes 32 MR WR weight rows x 32 MT WT tokens: WR x WT waves
  * of MR x MT tiles of 32 x 32 (v_mfma_f32_32x32x16_f16, A = tokens, B =
  * weight rows: lane l holds token / row l % 32, values 8 (l / 32) .. +7 of a
@@ -148,6 +173,30 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
         }
     };
 
+    /* the encoder's products add the same four parts of K in the same order
+     * in every tile, so that a text's embedding has the same bits alone and
+     * in a batch */
+    constexpr bool PO = EP <= EP_BIAS_GELU_SPLIT && WK == 1;
+    static_assert(EP > EP_BIAS_GELU_SPLIT || WK == 1 || WK == 4, "four parts");
+    v16f tot[PO ? MR : 1][PO ? MT : 1];
+    const int np = (ns + 3) / 4;
+    int next = np;
+#pragma unroll
+    for (int m = 0; m < (PO ? MR : 1); m++)
+#pragma unroll
+        for (int u = 0; u < (PO ? MT : 1); u++) tot[m][u] = (v16f){};
+    auto part = [&](int i) __attribute__((always_inline)) {
+        if (i != next) return;
+        next += np;
+#pragma unroll
+        for (int m = 0; m < (PO ? MR : 1); m++)
+#pragma unroll
+            for (int u = 0; u < (PO ? MT : 1); u++) {
+                tot[m][u] += acc[m][u];
+                acc[m][u] = (v16f){};
+            }
+    };
+
     Stg s0, s1;
     load(s0, 0);
     load(s1, 1);
@@ -155,13 +204,21 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
     __syncthreads();
     for (int i = 0; i < nsg; i += 2) {
         load(s0, i + 2);
+        if (PO) part(i);
         if (i < kn) compute(0);
         store(s1, 1);
         __syncthreads();
         load(s1, i + 3);
+        if (PO) part(i + 1);
         if (i + 1 < kn) compute(1);
         store(s0, 0);
         __syncthreads();
+    }
+    if constexpr (PO) {
+#pragma unroll
+        for (int i = 0; i < MR; i++)
+#pragma unroll
+            for (int u = 0; u < MT; u++) acc[i][u] = tot[i][u] + acc[i][u];
     }
     if constexpr (WK > 1) {
         /* the other groups' sums, in order (all stages are consumed) */
@@ -192,31 +249,14 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
         const int tb = t0 + (wt * MT + u) * 32 + 4 * h;   /* register r: token tb + 8 (r / 4) + r % 4 */
         float inv[16];
 #pragma unroll
-        for (int r = 0; r < 16; r++) inv[r] = x.inv[min(tb + 8 * (r >> 2) + (r & 3), a.T - 1)];
+        for (int r = 0; r < 16; r++) inv[r] = x.inv ? x.inv[min(tb + 8 * (r >> 2) + (r & 3), a.T - 1)] : x.inv_all;
 #pragma unroll
         for (int i = 0; i < MR; i++) {
             const int row = r0 + (wr * MR + i) * 32 + j;
             if (row >= a.R) continue;
-            const float bias = EP <= EP_BIAS_GELU ? a.bias[row] : 0.0f;
+            const float bias = EP <= EP_BIAS_GELU_SPLIT ? a.bias[row] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int t = tb + 8 * (r >> 2) + (r & 3);
-                if (t >= a.T) continue;
-                float o = acc[i][u][r] * inv[r];
-                if constexpr (EP == EP_STORE) {
-                } else if constexpr (EP == EP_ADD) {
-                    o = a.out[(size_t)t * a.ldo + row] + o;
-                } else if constexpr (EP == EP_BIAS) {
-                    o = o + bias;
-                } else if constexpr (EP == EP_BIAS_RES) {
-                    o = o + (bias + a.res[(size_t)t * a.ldr + row]);
-                } else {
-                    /* gelu (fast/lil_math.cpp:978-984) of row + bias */
-                    const float g = o + bias;
-                    o = 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));
-                }
-                a.out[(size_t)t * a.ldo + row] = o;
-            }
+            for (int r = 0; r < 16; r++) hg_emit<EP>(a, acc[i][u][r], inv[r], bias, tb + 8 * (r >> 2) + (r & 3), row);
         }
     }
 }
@@ -227,13 +267,16 @@ static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
     const int nrb = ((a.R + 32 * MR * WR - 1) / (32 * MR * WR) + 7) & ~7, nt = (a.T + 32 * MT * WT - 1) / (32 * MT * WT);
     const dim3 grid((unsigned)(nrb * nt)), blk(64 * WR * WT * WK);
 #define HG(E) hipLaunchKernelGGL((k_hgemm<MR, MT, WR, WT, WK, E>), grid, blk, 0, s, a, x)
-    switch (ep) {
-    case EP_BIAS: HG(EP_BIAS); break;
-    case EP_BIAS_RES: HG(EP_BIAS_RES); break;
-    case EP_BIAS_GELU: HG(EP_BIAS_GELU); break;
-    case EP_ADD: HG(EP_ADD); break;
-    default: HG(EP_STORE); break;
+    if constexpr (WK != 2) {
+        switch (ep) {
+        case EP_BIAS: HG(EP_BIAS); return;
+        case EP_BIAS_RES: HG(EP_BIAS_RES); return;
+        case EP_BIAS_GELU: HG(EP_BIAS_GELU); return;
+        case EP_BIAS_GELU_SPLIT: HG(EP_BIAS_GELU_SPLIT); return;
+        }
     }
+    if (ep == EP_ADD) HG(EP_ADD);
+    else HG(EP_STORE);
 #undef HG
 }
 
@@ -247,11 +290,22 @@ static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
  * 4096 x 4096, 150 tokens 32 / 34), and 32 x 32 with K in four parts for the
  * smallest (384 x 1536, 512 tokens 8.4 / 13) and for up to 32 tokens, where
  * the weights' stream is the bound (24576 x 4096, 13 tokens 50, 4.1 TB/s;
- * 64 x 64 60). */
+ * 64 x 64 60).
+ *
+ * The encoder's matrices are narrow, and every tile must add K's four parts
+ * in one order (PO above): 32 x 32 up to 384 such tiles (384 x 1536, 25
+ * tokens 9.0 / 64 x 64 16.8; 1152 x 384, 260 tokens 7.7 / 7.8, 512 tokens
+ * 9.5 / 8.0), 64 x 64 above (4096 tokens: 1152 x 384 24.3, 384 x 384 15.6,
+ * 1536 x 384 25.9, 384 x 1536 35.4; 128 x 128 25.0, 30.7, 30.0, 50.2), and
+ * 128 x 128 once it gives every CU two. */
 int lg_hgemm(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
 {
     auto wgs = [&](int tr, int tt) { return (long)((a.R + tr - 1) / tr) * ((a.T + tt - 1) / tt); };
-    if (a.T <= 32) hgemm_launch<1, 1, 1, 1, 4>(a, x, ep, s);
+    if (ep <= EP_BIAS_GELU_SPLIT) {
+        if (wgs(32, 32) <= 384) hgemm_launch<1, 1, 1, 1, 4>(a, x, ep, s);
+        else if (wgs(128, 128) >= 512) hgemm_launch<2, 2, 2, 2, 1>(a, x, ep, s);
+        else hgemm_launch<1, 1, 2, 2, 1>(a, x, ep, s);
+    } else if (a.T <= 32) hgemm_launch<1, 1, 1, 1, 4>(a, x, ep, s);
     else if (wgs(128, 128) >= 256) hgemm_launch<2, 2, 2, 2, 1>(a, x, ep, s);
     else if (wgs(128, 64) >= 384) hgemm_launch<2, 1, 2, 2, 1>(a, x, ep, s);
     else if (wgs(128, 64) >= 224) hgemm_launch<2, 1, 2, 2, 2>(a, x, ep, s);

@@ -1,0 +1,60 @@
+"""The encoder's F16 path where it can go wrong: attention at the edges of its
+16-query blocks and 32-key steps, every head width, a wave or a workgroup to
+a query block, alone and in a batch bit for bit (other tiles of the products), and activations split by their producer (bounds of the weights)
+or from each token's own maximum (F32 producers, bounds that are none)."""
+import zlib
+
+import numpy as np
+import pytest
+
+from ligguf_amd import encode
+from ligguf_amd.bert import BERT_TINY, Bert, HostBert
+from ligguf_amd.lib import F16, F32
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 13, 14, 15, 30, 31, 62, 63, 125, 126, 127, 158, 159, 257]      # with CLS and SEP: at the blocks' and steps' ends
+REL = 2e-5   # fp32 sums in another order, activations to 2^-21: the bar of the encoder tests
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.asarray(a, np.float64) - b) / np.linalg.norm(np.asarray(b, np.float64)))
+
+
+def texts(cfg, lengths):
+    return [np.random.default_rng(n).integers(5, cfg.vocab, n).astype(np.int32) for n in lengths]
+
+
+@pytest.mark.parametrize("hd", [16, 32, 48, 64, 80, 96, 112, 128])
+def test_attention_edges(gpu, oracle, hd):
+    hb = HostBert.synthetic(BERT_TINY.with_(n_heads=2, n_embed=2 * hd, n_ff=416, n_layers=2, n_context=288,
+                                            layer_type=F16, embd_type=F16))
+    dev = Bert(0)
+    dev.load(hb, 4096)
+    seqs = texts(hb.cfg, LENGTHS)
+    one = np.stack([dev.embed(s) for s in seqs])
+    many = dev.embed_batch(seqs * 3)
+    dev.close()
+    for i, s in enumerate(seqs):
+        ref = oracle.bert_embed(hb, s)
+        assert rel(one[i], ref) < REL, (hd, len(s), rel(one[i], ref))
+    assert np.array_equal(many.view(np.uint32), np.tile(one, (3, 1)).view(np.uint32))
+
+
+@pytest.mark.parametrize("f32", [("attn_q", "attn_k", "attn_v", "ffn_up"), ("attn_v",), ("attn_output", "ffn_down"), ("ffn_up",)])
+def test_split_follows_the_producer(gpu, oracle, f32):
+    cfg = BERT_TINY.with_(layer_type=F16, embd_type=F16)
+    hb = HostBert.synthetic(cfg)
+    for name, (t, rows, cols, _) in list(hb.weights.items()):
+        if name.split(".")[-2] in f32:
+            hb.weights[name] = (F32, rows, cols, encode.random_tensor(F32, 3, zlib.crc32(name.encode()), rows, cols, cfg.sigma))
+    # LayerNorm outputs, and so the bounds, of very different sizes
+    for l, m in enumerate((1e-6, 1e4, 1.0, 30.0)):
+        for n in ("attn_output_norm.weight", "attn_output_norm.bias"):
+            if l < cfg.n_layers:
+                hb.vectors[f"blk.{l}.{n}"] = hb.vectors[f"blk.{l}.{n}"] * np.float32(m)
+    dev = Bert(0)
+    dev.load(hb)
+    for s in texts(hb.cfg, [2, 40]):
+        assert rel(dev.embed(s), oracle.bert_embed(hb, s)) < REL
+    dev.close()
