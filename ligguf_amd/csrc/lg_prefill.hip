@@ -2055,275 +2055,6 @@ int lg_prefill_gemm(int wtype, const uint8_t* W, uint32_t rsz, int rows, int col
     }
 }
 
-/* ------------------------------------------------------------------ */
-/* causal attention on fp16 MFMA: 16 query tokens x one KV head          */
-/* ------------------------------------------------------------------ */
-/* One workgroup per (16-token query block, KV head g), one wave per query
- * head of the group (and, up to 4 query heads per KV head, per half of the
- * key blocks: the halves merge at the end).  Per block of 16 key positions
- * the K and V rows come from the fp16 cache into LDS, and each wave
- * computes the scores and the output with an online softmax per query
- * column in log2 units (the decode step's attention does the same per lane
- * group).  A query's own key and value are its fp32 k/v (the cache holds
- * them in fp16), as in the token-sequential step: in the key block holding
- * a query's position its score is recomputed from the fp32 k row, and its
- * value enters as the fp16 row through the MFMA plus p (v32 - v16).  Key
- * positions past a query's own are masked.
- *
- * The products run on fp16 MFMA (v_mfma_f32_16x16x16_f16, fp32
- * accumulation): the cache rows are fp16 already, and each fp32
- * operand goes in as two fp16 parts, x = hi + lo (hi = fp16(x), lo =
- * fp16(x - hi)), so q.k = hi.k + lo.k and p.v = hi.v + lo.v keep ~22 bits of
- * every fp32 operand (each fp16 x fp16 product is exact in fp32).  p <= 1 is
- * scaled by 2^15 before the split, so p down to 2^-29 stays a normal fp16,
- * and the sums are unscaled at the end.  K is staged in LDS as it is
- * stored ([key][dim], rows padded 16 B against bank conflicts), V transposed
- * ([dim][key]): an MFMA lane takes 4 consecutive keys of one dim.
- *   S^T[key][q] = sum_d K[key][d] Q[q][d]   A = K, B = Q^T (16 dims a step)
- *   O^T[d][q]  += sum_key V^T[d][key] P^T[key][q]   A = V^T, B = P^T
- * P^T is the D layout of S^T (lane (g, q) holds keys 4g..4g+3), so it feeds
- * the second product without a transpose.  Only fp32 rounding differs from
- * the token-sequential step (sum orders, ~2^-22 per operand). */
-template <int HD, int NREP, int SPLIT>
-__global__ __launch_bounds__(64 * NREP * SPLIT) void k_pf_attn_h(const float* __restrict__ qkv, int qstride, int n_embed,
-                                                         int kv_dim, const uint16_t* __restrict__ kc,
-                                                         const uint16_t* __restrict__ vc, int pos0, int T,
-                                                         float* __restrict__ att)
-{
-    static_assert(HD % 16 == 0 && HD <= 256, "16-dim output tiles");
-    constexpr int NT = 64 * NREP * SPLIT, NTL = HD / 16, KST = HD + 8, VTS = 20, OST = HD + 4;
-    constexpr float PS = 32768.0f;
-    __shared__ __attribute__((aligned(16))) _Float16 s_kh[SPLIT][16 * KST];   /* K[key][d] */
-    __shared__ __attribute__((aligned(16))) _Float16 s_vt[SPLIT][HD * VTS];   /* V^T[d][key] */
-    __shared__ __attribute__((aligned(16))) float s_k32[16 * OST];    /* fp32 k / v of the block's 16 tokens */
-    __shared__ __attribute__((aligned(16))) float s_v32[16 * OST];
-    const int qb = blockIdx.x, g = blockIdx.y;
-    const int tid = threadIdx.x, lane = tid & 63, r = (tid >> 6) % NREP, half = (tid >> 6) / NREP;
-    const _Float16* __restrict__ s_k = s_kh[half];
-    const _Float16* __restrict__ s_v = s_vt[half];
-    const int col = lane & 15, grp = lane >> 4;
-    const int t0 = qb * 16, tq = t0 + col, tqc = min(tq, T - 1);
-    const int qpos = pos0 + tq;
-    const int last = pos0 + min(t0 + 15, T - 1);   /* last key position this block reads */
-    const float scale2 = 1.44269504088896341f / sqrtf((float)HD);
-
-    /* B operand of S^T: Q[tq][16j + 4 grp + i], fp32 and as hi + lo */
-    float qf[NTL][4];
-    v4h qh[NTL], ql[NTL];
-    const float* qrow = qkv + (size_t)tqc * qstride + (size_t)(g * NREP + r) * HD;
-#pragma unroll
-    for (int j = 0; j < NTL; j++) {
-        const float4 v = *(const float4*)(qrow + 16 * j + 4 * grp);
-        qf[j][0] = v.x; qf[j][1] = v.y; qf[j][2] = v.z; qf[j][3] = v.w;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const _Float16 h = (_Float16)qf[j][i];
-            qh[j][i] = h;
-            ql[j][i] = (_Float16)(qf[j][i] - (float)h);
-        }
-    }
-    for (int i = tid; i < 16 * HD; i += NT) {
-        const int tt = i / HD, d = i % HD;
-        const float* row = qkv + (size_t)min(t0 + tt, T - 1) * qstride;
-        s_k32[tt * OST + d] = row[n_embed + g * HD + d];
-        s_v32[tt * OST + d] = row[n_embed + kv_dim + g * HD + d];
-    }
-
-    v4f o[NTL];
-#pragma unroll
-    for (int t = 0; t < NTL; t++) o[t] = (v4f){0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.0f;   /* l: this lane group's keys only, summed at the end */
-    const int nkb = last / 16 + 1, nit = (nkb + SPLIT - 1) / SPLIT;
-    constexpr int NPC = SPLIT * 16 * (HD / 8), NSTG = (NPC + NT - 1) / NT;
-    /* the K/V pieces of the next step (piece i: 8 dims of one key of one
-     * half's block), loaded while this step computes */
-    struct Pieces {
-        uint4 k[NSTG], v[NSTG];
-    };
-    auto stage_load = [&](int it) {
-        Pieces P;
-#pragma unroll
-        for (int u = 0; u < NSTG; u++) {
-            const int i = min(tid + u * NT, NPC - 1);
-            const int hb = i / (16 * (HD / 8)), kk = (i / (HD / 8)) % 16, d8 = (i % (HD / 8)) * 8;
-            const size_t off = (size_t)min((it * SPLIT + hb) * 16 + kk, last) * kv_dim + (size_t)g * HD + d8;
-            P.k[u] = *(const uint4*)(kc + off);
-            P.v[u] = *(const uint4*)(vc + off);
-        }
-        return P;
-    };
-    Pieces pc = stage_load(0);
-    for (int it = 0; it < nit; it++) {
-        __syncthreads();   /* the previous step's tiles are consumed */
-#pragma unroll
-        for (int u = 0; u < NSTG; u++) {
-            const int i = tid + u * NT;
-            if (NSTG * NT == NPC || i < NPC) {   /* (every thread has a piece when the pieces divide evenly) */
-                const int hb = i / (16 * (HD / 8)), kk = (i / (HD / 8)) % 16, d8 = (i % (HD / 8)) * 8;
-                *(uint4*)&s_kh[hb][kk * KST + d8] = pc.k[u];
-                const uint4 vv = pc.v[u];
-                uint16_t* vt = (uint16_t*)s_vt[hb] + d8 * VTS + kk;
-                vt[0] = (uint16_t)(vv.x & 0xffffu);
-                vt[VTS] = (uint16_t)(vv.x >> 16);
-                vt[2 * VTS] = (uint16_t)(vv.y & 0xffffu);
-                vt[3 * VTS] = (uint16_t)(vv.y >> 16);
-                vt[4 * VTS] = (uint16_t)(vv.z & 0xffffu);
-                vt[5 * VTS] = (uint16_t)(vv.z >> 16);
-                vt[6 * VTS] = (uint16_t)(vv.w & 0xffffu);
-                vt[7 * VTS] = (uint16_t)(vv.w >> 16);
-            }
-        }
-        __syncthreads();
-        pc = stage_load(min(it + 1, nit - 1));
-        const int kb = it * SPLIT + half;
-        if (kb >= nkb) continue;   /* the other half's last block (wave-uniform) */
-
-        v4f sa = (v4f){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < NTL; j++) {
-            const v4h a = *(const v4h*)(s_k + col * KST + 16 * j + 4 * grp);
-            sa = __builtin_amdgcn_mfma_f32_16x16x16f16(a, qh[j], sa, 0, 0, 0);
-            sa = __builtin_amdgcn_mfma_f32_16x16x16f16(a, ql[j], sa, 0, 0, 0);
-        }
-        float sv[4] = {sa[0], sa[1], sa[2], sa[3]};
-        /* the block holds some query's own position: exact fp32 scores */
-        const bool diag = kb * 16 + 15 >= pos0 + t0 && kb * 16 <= pos0 + t0 + 15;
-        const int own = qpos - kb * 16;   /* 0..15 when this lane's query owns a key here */
-        if (diag) {
-            float e = 0.0f;
-#pragma unroll
-            for (int j = 0; j < NTL; j++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) e = __builtin_fmaf(qf[j][i], s_k32[col * OST + 16 * j + 4 * grp + i], e);
-            e += lg_partner<4>(e);
-            e += lg_partner<5>(e);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (own == 4 * grp + i) sv[i] = e;
-        }
-        float bm = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            sv[i] = kb * 16 + 4 * grp + i > qpos ? -INFINITY : sv[i] * scale2;
-            bm = fmaxf(bm, sv[i]);
-        }
-        bm = fmaxf(bm, lg_partner<4>(bm));
-        bm = fmaxf(bm, lg_partner<5>(bm));
-        const float mn = fmaxf(m, bm);   /* finite: key 0 is in every query's range */
-        const float alpha = __builtin_amdgcn_exp2f(m - mn);
-        float pw[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) pw[i] = __builtin_amdgcn_exp2f(sv[i] - mn);
-        l = __builtin_fmaf(l, alpha, (pw[0] + pw[1]) + (pw[2] + pw[3]));
-        m = mn;
-        float pown = 0.0f;   /* p of the own key, broadcast to the column's four lane groups */
-        if (diag) {
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                if (own == 4 * grp + i) pown = pw[i];
-            pown += lg_partner<4>(pown);
-            pown += lg_partner<5>(pown);
-        }
-        /* P^T operand: the lane's keys 4 grp..+3, scaled, as hi + lo */
-        v4h ph, pl;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float ps = pw[i] * PS;
-            const _Float16 h = (_Float16)ps;
-            ph[i] = h;
-            pl[i] = (_Float16)(ps - (float)h);
-        }
-#pragma unroll
-        for (int t = 0; t < NTL; t++) {
-            o[t] *= alpha;
-            const v4h a = *(const v4h*)(s_v + (16 * t + col) * VTS + 4 * grp);
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, ph, o[t], 0, 0, 0);
-            o[t] = __builtin_amdgcn_mfma_f32_16x16x16f16(a, pl, o[t], 0, 0, 0);
-        }
-        if (diag && own >= 0 && own < 16) {
-            const float pso = pown * PS;
-#pragma unroll
-            for (int t = 0; t < NTL; t++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int d = 16 * t + 4 * grp + i;
-                    o[t][i] = __builtin_fmaf(pso, s_v32[col * OST + d] - (float)s_v[d * VTS + own], o[t][i]);
-                }
-        }
-    }
-    if constexpr (SPLIT == 2) {
-        /* the second half's (m, l, o) into the first half's lanes */
-        __shared__ float s_x[NREP][2 + 4 * NTL][64];
-        if (half == 1) {
-            s_x[r][0][lane] = m;
-            s_x[r][1][lane] = l;
-#pragma unroll
-            for (int t = 0; t < NTL; t++)
-#pragma unroll
-                for (int i = 0; i < 4; i++) s_x[r][2 + 4 * t + i][lane] = o[t][i];
-        }
-        __syncthreads();
-        if (half == 1) return;
-        const float m1 = s_x[r][0][lane], mx = fmaxf(m, m1);
-        const float a0 = __builtin_amdgcn_exp2f(m - mx), a1 = __builtin_amdgcn_exp2f(m1 - mx);
-        l = lg_fma2(l, a0, s_x[r][1][lane], a1);
-#pragma unroll
-        for (int t = 0; t < NTL; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) o[t][i] = lg_fma2(o[t][i], a0, s_x[r][2 + 4 * t + i][lane], a1);
-    }
-    l += lg_partner<4>(l);
-    l += lg_partner<5>(l);
-    if (tq < T) {
-        const float inv = 1.0f / (l * PS);
-        float* out = att + (size_t)tq * n_embed + (size_t)(g * NREP + r) * HD;
-#pragma unroll
-        for (int t = 0; t < NTL; t++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) out[16 * t + 4 * grp + i] = o[t][i] * inv;
-    }
-}
-
-int lg_prefill_attn_supported(int head_dim, int nrep)
-{
-    return (head_dim == 48 || head_dim == 64 || head_dim == 128) && nrep >= 1 && nrep <= 8;
-}
-
-static int launch_attn(const PfModel& M, const float* qkv, int qs, const uint16_t* kc, const uint16_t* vc, int T,
-                       int pos0, float* att, hipStream_t s)
-{
-    const int nrep = M.n_heads / M.n_kv;
-    if (!lg_prefill_attn_supported(M.head_dim, nrep)) {
-        lg_set_error("prefill attention: head_dim %d with %d query heads per KV head", M.head_dim, nrep);
-        return LG_ERR_TYPE;
-    }
-    const dim3 grid((T + 15) / 16, M.n_kv);
-    /* two halves of the key blocks per query head up to 4 query heads per
-     * KV head (8 waves); one at 8 (8 waves already) */
-#define PFA(HD, NR)                                                                                          \
-    hipLaunchKernelGGL((k_pf_attn_h<HD, NR, (NR <= 4 ? 2 : 1)>), grid, dim3(64 * NR * (NR <= 4 ? 2 : 1)), 0, s, \
-                       qkv, qs, M.n_embed, M.kv_dim, kc, vc, pos0, T, att)
-#define PFA_HD(HD)                    \
-    switch (nrep) {                   \
-    case 1: PFA(HD, 1); break;        \
-    case 2: PFA(HD, 2); break;        \
-    case 3: PFA(HD, 3); break;        \
-    case 4: PFA(HD, 4); break;        \
-    case 5: PFA(HD, 5); break;        \
-    case 6: PFA(HD, 6); break;        \
-    case 7: PFA(HD, 7); break;        \
-    default: PFA(HD, 8); break;       \
-    }
-    switch (M.head_dim) {
-    case 48: PFA_HD(48); break;
-    case 64: PFA_HD(64); break;
-    default: PFA_HD(128); break;
-    }
-#undef PFA_HD
-#undef PFA
-    return lg_check_launch("prefill attention");
-}
-
 /* one pass's quantized activation of every token into the trace, as the
  * reference's blocks (block_q8_K: d, qs[256], bsums[16]; block_q8_0: fp16 d,
  * qs[32]): block b of token t */
@@ -2406,7 +2137,7 @@ int lg_prefill_layers(const PfModel& M, PfBuffers& B, int T, int pos0, hipStream
         hipLaunchKernelGGL(k_pf_qk_rope_kv, dim3((waves + 3) / 4, T), dim3(256), 0, s, B.qkv, qs, ne, kvd, L.q_norm,
                            L.k_norm, M.n_heads, M.n_kv, M.head_dim, M.rope_dim, pos0, M.rope_freq, M.eps, kc, vc);
         if ((rc = lg_check_launch("prefill qk-norm/rope/kv"))) return rc;
-        if ((rc = launch_attn(M, B.qkv, qs, kc, vc, T, pos0, B.att, s))) return rc;
+        if ((rc = lg_prefill_attn(M, B.qkv, qs, kc, vc, T, pos0, B.att, B.attp, s))) return rc;
         if ((rc = quant(fam(L.ao), B.att, nullptr, ne, 4 * l + 1))) return rc;
         if ((rc = gemm(L.ao, ne, B.x, ne, 1))) return rc;
         /* FFN branch */
