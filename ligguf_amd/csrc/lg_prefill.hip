@@ -962,31 +962,65 @@ static bool pf_gemm16()
 
 bool lg_prefill_gemm16() { return pf_gemm16(); }
 
-/* Tile (rows x tokens, K parts) of the 32 x 32 product kernels by the number
- * of 32 x 32 output tiles.  A wave walks its part of K block by block, each
- * waiting on loads that the block before issued, so its time is the number
- * of blocks: where the wide tile would leave most of the 1024 SIMDs without
- * a wave, smaller workgroups with K in more parts finish sooner, though they
- * unpack each weight for fewer tokens.  Measured (us at the tile taken / at
- * 128 x 64 with K in two parts, the former choice):
- *   24576 x 4096, 512 tokens   Q4_K 170 / 178  (12288 tiles)
- *    4096 x 4096, 512 tokens   Q4_K 27 (both)  (2048: a workgroup a CU, K in two)
- *    4096 x 12288, 200 tokens  Q4_K 50 / 64, Q8_0 170 / 194, Q1_G 84 / 133  (896)
- *    6144 x 4096, 77 tokens    Q4_K 20 / 24, Q1_G 30 / 47  (576)
- *    4096 x 12288, 77 tokens   Q4_K 30 / 62, Q6_K 55 / 109, Q8_0 92 / 196  (384)
- *    4096 x 12288, 16 tokens   Q4_K 21 / 60, Q6_K 35 / 109, Q1_G 35 / 130  (128)
- *     600 x 2048, 96 tokens    Q4_K 6.7 / 14, Q6_K 9.3 / 22  (57)
- * and on the other side of each line 24576 x 4096, 77 tokens (2304) Q4_K 45
- * at 128 x 64, 48 at 64 x 32; 4096 x 4096, 200 tokens (896) Q4_K 20 with K
- * in two parts, 24 in four. */
-enum { PF_T128x64, PF_T128x64_K2, PF_T64x32_K2, PF_T64x32_K4, PF_T32x32_K4 };
-static int pf_tile(int rows, int T)
+/* Tiles of the 32 x 32 product kernels: rows x tokens of a workgroup and the
+ * parts of K its wave groups take, and what a workgroup costs -- to start,
+ * and per 256 values of K alone on its CU or with a second one beside it
+ * (then both take `pair` together; the 8-wave workgroups of 128 x 64 in two
+ * parts and 64 x 32 in four have no room beside them and take twice their
+ * time).  A CU holds ceil(workgroups / 256) of them in turn, and a part of K
+ * that has nothing to compute still walks its steps, so
+ *   cost = p start + steps parts (p / 2 pair + p % 2 alone)
+ * gives the tile: smaller workgroups fill more CUs and walk less of K each,
+ * larger ones unpack a weight for more tokens and write each sum once.  The
+ * table (units of about 0.07 us for Q4_K, 0.25 for Q8_0) is one least
+ * regret over 12 row forms, 96 to 24576 rows, 256 to 12544 columns and 2 to
+ * 512 tokens, each tile timed with weights from HBM (3013 shapes): the tile
+ * taken is 0.4 % above the fastest in the mean, and none is slower than 128 x
+ * 64 with K in two parts up to 256 workgroups and from 1024 columns, the
+ * choice before these tiles, which is 35 % above the fastest.  us at the
+ * tile taken / at that choice:
+ *    4096 x 4096, 257..448 tokens  Q4_K 27..33 (both; 64 x 32 in two 31..43), Q5_K 37..42 (both; 42..58)
+ *    4096 x 12288, 77 tokens       Q4_K 35 / 72, Q6_K 59 / 117, Q8_0 96 / 206
+ *    6144 x 4096, 77 tokens        Q4_K 21 / 25, Q1_G 30 / 47
+ *    4096 x 12288, 16 tokens       Q4_K 23 / 64, Q6_K 36 / 111, Q1_G 36 / 130
+ *    4096 x 512, 200 tokens        Q6_K 9.4 (128 x 64 unsplit; 64 x 32 in two 11.9) */
+struct PfTile {
+    int rows, tokens, parts, start, alone, pair;
+};
+enum { PF_T128x64, PF_T128x64_K2, PF_T64x32_K2, PF_T64x32_K4, PF_T32x32_K4, PF_TILES };
+static constexpr PfTile pf_tiles[PF_TILES] = {
+    {128, 64, 1, 24, 20, 30}, {128, 64, 2, 32, 16, 35}, {64, 32, 2, 20, 8, 13}, {64, 32, 4, 30, 6, 13}, {32, 32, 4, 18, 5, 7}};
+
+static int pf_tile(int rows, int cols, int T)
 {
-    const long n32 = (long)((rows + 31) / 32) * ((T + 31) / 32);
-    if (n32 < 256) return PF_T32x32_K4;
-    if (n32 < 500) return PF_T64x32_K4;
-    if (n32 < 1800) return PF_T64x32_K2;
-    return (long)((rows + 127) / 128) * ((T + 63) / 64) <= 256 ? PF_T128x64_K2 : PF_T128x64;
+    int best = 0;
+    long low = 0;
+    for (int i = 0; i < PF_TILES; i++) {
+        const PfTile& t = pf_tiles[i];
+        /* the launch pads the row blocks to a multiple of 8 (the XCDs) */
+        const long wgs = (long)(((rows + t.rows - 1) / t.rows + 7) & ~7) * ((T + t.tokens - 1) / t.tokens);
+        const long p = (wgs + 255) / 256, steps = ((cols + 255) / 256 + t.parts - 1) / t.parts;
+        const long cost = p * t.start + steps * t.parts * (p / 2 * t.pair + p % 2 * t.alone);
+        if (i == 0 || cost < low) {
+            low = cost;
+            best = i;
+        }
+    }
+    return best;
+}
+
+/* (tests) the tile the int8 GEMMs take for rows x cols times T tokens */
+extern "C" int lg_prefill_tile(int rows, int cols, int T, int* tile_rows, int* tile_tokens, int* k_parts)
+{
+    if (rows <= 0 || cols <= 0 || T <= 0 || !tile_rows || !tile_tokens || !k_parts) {
+        lg_set_error("prefill tile: bad arguments");
+        return LG_ERR_ARG;
+    }
+    const PfTile& t = pf_tiles[pf_tile(rows, cols, T)];
+    *tile_rows = t.rows;
+    *tile_tokens = t.tokens;
+    *k_parts = t.parts;
+    return LG_OK;
 }
 
 template <int WT, int RW, int KS, int TT>
@@ -1004,7 +1038,7 @@ static int gemm_k32(const uint8_t* W, uint32_t rsz, int rows, int cols, const Pf
                     int accumulate, hipStream_t s)
 {
 #define K32(RW, KS, TT) k32_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
-    switch (pf_tile(rows, T)) {
+    switch (pf_tile(rows, cols, T)) {
     case PF_T128x64: K32(4, 1, 64); break;
     case PF_T128x64_K2: K32(4, 2, 64); break;
     case PF_T64x32_K2: K32(2, 2, 32); break;
@@ -1936,7 +1970,7 @@ static int gemm_b32x(const uint8_t* W, uint32_t rsz, int rows, int cols, const P
                      int accumulate, hipStream_t s)
 {
 #define B32X(RW, KS, TT) b32x_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
-    switch (pf_tile(rows, T)) {
+    switch (pf_tile(rows, cols, T)) {
     case PF_T128x64: B32X(4, 1, 64); break;
     case PF_T128x64_K2: B32X(4, 2, 64); break;
     case PF_T64x32_K2: B32X(2, 2, 32); break;

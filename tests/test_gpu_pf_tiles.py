@@ -2,17 +2,23 @@
 batched prefill picks -- 128 x 64, 64 x 32 and 32 x 32 with K in one, two or
 four parts, fewer blocks of K than parts, ends of rows and tokens -- against
 float64 over the same quantized operands."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
 
 from ligguf_amd import encode, ops
-from ligguf_amd.lib import Q1_0, Q1_G, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, TYPE_NAMES, row_size
+from ligguf_amd.lib import Q1_0, Q1_G, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, TYPE_NAMES, load, row_size
 
 pytestmark = pytest.mark.gpu
 
-# rows, width, tokens: 32 x 32 | 64 x 32, K in 4 | 64 x 32, K in 2 | 128 x 64, K in 2 | 128 x 64
-SHAPES = [(33, 256, 1), (600, 2304, 95), (4090, 1280, 33), (4097, 512, 65), (6145, 768, 100), (3970, 1280, 449), (12289, 512, 165)]
+# rows, width, tokens, the tile taken (rows x tokens, parts of K): ends of rows and tokens, one step of K in two parts,
+# as many steps as parts and fewer, an uneven last part
+SHAPES = [(33, 256, 1, (64, 32, 2)), (600, 2304, 95, (32, 32, 4)), (4090, 1280, 33, (32, 32, 4)), (65, 768, 40, (32, 32, 4)),
+          (4097, 512, 65, (64, 32, 2)), (4065, 1280, 100, (64, 32, 2)), (4033, 1792, 97, (64, 32, 4)),
+          (3970, 2304, 449, (128, 64, 2)), (6145, 768, 100, (128, 64, 1)), (3970, 1280, 449, (128, 64, 1)),
+          (12289, 512, 165, (128, 64, 1))]
 TYPES = [Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, Q1_0, Q1_G]
 
 
@@ -28,8 +34,10 @@ def activations(x, kq):
 
 
 @pytest.mark.parametrize("wt", TYPES, ids=[TYPE_NAMES[t] for t in TYPES])
-@pytest.mark.parametrize("R,n,T", SHAPES)
-def test_tiles(gpu, wt, R, n, T):
+@pytest.mark.parametrize("R,n,T,tile", SHAPES)
+def test_tiles(gpu, wt, R, n, T, tile):
+    got = [C.c_int() for _ in range(3)]
+    assert load().lg_prefill_tile(R, n, T, *(C.byref(o) for o in got)) == 0 and tuple(o.value for o in got) == tile
     rsz = row_size(wt, n)
     distinct = min(R, 512)   # encoding is host work: the rows repeat, with a stride that no tile edge divides
     rows = encode.random_tensor(wt, R + n, wt, distinct, n).reshape(distinct, rsz)
