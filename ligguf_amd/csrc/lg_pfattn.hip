@@ -187,10 +187,10 @@ __global__ __launch_bounds__(64 * NREP * (NREP <= 4 ? 2 : 1)) void k_pf_attn(
      * unit took about a cycle for each (20 tokens after 100: 17.4 -> 15.2 us;
      * 512 after none 26.5 -> 21.8). */
     constexpr int DW = C::DW, PR = DW + 4;
-    auto rows = [&](v4f* R, int off) __attribute__((always_inline)) {
+    auto rows = [&](v4f* R, int off, int tb) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < C::NP * C::NI; i++)
-            R[i] = *(const v4f*)(qkv + (size_t)min(t0 + i % C::NI * C::RPI + lane / C::LPR, T - 1) * qstride + off +
+            R[i] = *(const v4f*)(qkv + (size_t)min(tb + i % C::NI * C::RPI + lane / C::LPR, T - 1) * qstride + off +
                                  i / C::NI * DW + lane % C::LPR * 4);
     };
     auto wave_sync = [] __attribute__((always_inline)) {   /* the wave's LDS writes before its other lanes' reads */
@@ -205,8 +205,8 @@ __global__ __launch_bounds__(64 * NREP * (NREP <= 4 ? 2 : 1)) void k_pf_attn(
     float eown = 0.0f;
     {
         v4f Rq[C::NP * C::NI], Rk[C::NP * C::NI];
-        rows(Rq, (g * NREP + r) * HD);
-        rows(Rk, n_embed + g * HD);
+        rows(Rq, (g * NREP + r) * HD, t0);
+        rows(Rk, n_embed + g * HD, t0);
         float* const w = (float*)(s_raw + (size_t)wave * (C::LDS / (NREP * SPLIT) & ~15));
         float* const wr = w + lane / C::LPR * PR + lane % C::LPR * 4;
         const float* const rd = w + col * PR + 8 * h;
@@ -313,8 +313,14 @@ __global__ __launch_bounds__(64 * NREP * (NREP <= 4 ? 2 : 1)) void k_pf_attn(
         __syncthreads();
     }
     l += lg_partner<5>(l);
-    v4f Rv[C::NP * C::NI];   /* the own values, in rows */
-    rows(Rv, n_embed + kv_dim + g * HD);
+    /* the own values, in rows.  Their addresses are worked out again: taken
+     * for the same expressions as the queries', they lived through the key
+     * loop, which at 128 dims has no registers to spare, and 112 bytes a lane
+     * went to scratch -- set up on the stream inside an engine's first prompt */
+    v4f Rv[C::NP * C::NI];
+    int te = t0;
+    __asm__ volatile("" : "+s"(te));
+    rows(Rv, n_embed + kv_dim + g * HD, te);
     if constexpr (SPLIT == 2) {
         /* the second half's (c, l, o) into the first half's lanes */
         float* x = (float*)s_raw + (size_t)r * (2 + 16 * NTO) * 64 + lane;   /* (the tiles are consumed) */
