@@ -1005,9 +1005,9 @@ static int prefill_buffers(lg_ctx* c)
     if ((rc = dalloc(c, (void**)&B.x, (size_t)tmax * ne * 4))) return rc;
     if ((rc = dalloc(c, (void**)&B.qkv, (size_t)tmax * qs * 4))) return rc;
     if ((rc = dalloc(c, (void**)&B.att, (size_t)tmax * ne * 4))) return rc;
-    if ((rc = dalloc(c, (void**)&B.ug, (size_t)tmax * 2 * nff * 4))) return rc;
-    const size_t np = lg_prefill_attn_part(c->n_context, c->n_heads, c->n_kv_heads, c->head_dim);
-    if (np && (rc = dalloc(c, (void**)&B.attp, np * 4))) return rc;
+    /* up|gate's output; the attention before it keeps its partials there */
+    B.ug_floats = std::max((size_t)tmax * 2 * nff, lg_prefill_attn_part(c->n_context, c->n_heads, c->n_kv_heads, c->head_dim));
+    if ((rc = dalloc(c, (void**)&B.ug, B.ug_floats * 4))) return rc;
     if (c->pf_fam & 1) {   /* Q8_K: quants, a scale and 16 bsums per 256 values */
         if ((rc = dalloc(c, (void**)&B.qk.qs, (size_t)tmax * wide))) return rc;
         if ((rc = dalloc(c, (void**)&B.qk.d, wide / 256 * tmax * 4))) return rc;

@@ -413,12 +413,7 @@ __global__ __launch_bounds__(256) void k_pf_attn_merge(const float* __restrict__
  * layers, 3 tokens after 6000, 367 us with 1024 keys a chunk, 342 with 512,
  * 329 with 256, 332 with 128; 512 tokens after none 833 with 512, 829 with
  * 256. */
-#ifndef PF_ATT_WGS
-#define PF_ATT_WGS 256
-#endif
-#ifndef PF_ATT_KEYS
-#define PF_ATT_KEYS 256
-#endif
+constexpr int PF_ATT_WGS = 256, PF_ATT_KEYS = 256;
 static int pf_attn_split(int T, int keys, int n_kv)
 {
     return std::max(1, std::min(PF_ATT_WGS / ((T + 31) / 32 * n_kv), keys / PF_ATT_KEYS));
@@ -437,7 +432,7 @@ int lg_prefill_attn_supported(int head_dim, int nrep)
 }
 
 int lg_prefill_attn(const PfModel& M, const float* qkv, int qs, const uint16_t* kc, const uint16_t* vc, int T, int pos0,
-                    float* att, float* part, hipStream_t s)
+                    float* att, float* part, size_t part_floats, hipStream_t s)
 {
     const int nrep = M.n_heads / M.n_kv;
     if (!lg_prefill_attn_supported(M.head_dim, nrep)) {
@@ -445,7 +440,9 @@ int lg_prefill_attn(const PfModel& M, const float* qkv, int qs, const uint16_t* 
         return LG_ERR_TYPE;
     }
     const int keys = pos0 + T;
-    int ns = part ? pf_attn_split(T, keys, M.n_kv) : 1;
+    /* chunks that the partials have room for */
+    const size_t room = part_floats / (T * pf_part_row(M.n_heads, M.head_dim));
+    int ns = (int)std::min<size_t>(pf_attn_split(T, keys, M.n_kv), std::max<size_t>(room, 1));
     const int ck = ((keys + ns - 1) / ns + 127) & ~127;   /* whole tiles of both halves */
     ns = (keys + ck - 1) / ck;
     if (ns == 1) part = nullptr;

@@ -58,8 +58,8 @@ struct PfBuffers {
     float* x;        /* [tmax][n_embed] residual stream */
     float* qkv;      /* [tmax][n_embed + 2 kv_dim] */
     float* att;      /* [tmax][n_embed] */
-    float* attp;     /* attention partials, lg_prefill_attn_part() floats (NULL when none are needed) */
-    float* ug;       /* [tmax][2 n_ff] */
+    float* ug;       /* [tmax][2 n_ff]; before that the attention's partials */
+    size_t ug_floats;
     PfQ8K qk;        /* Q8_K form, width up to n_ff (qs NULL when no matrix takes it) */
     PfQ8K q0;        /* Q8_0 form (likewise) */
     PfQ8K qf;        /* F32 form (likewise; only f and tld) */
@@ -81,9 +81,10 @@ int lg_prefill_attn_supported(int head_dim, int nrep);
 size_t lg_prefill_attn_part(int n_ctx, int n_heads, int n_kv, int head_dim);
 /* causal attention of T tokens at pos0.. (lg_pfattn.hip): qkv rows of qs
  * floats as the rope kernel leaves them, the layer's cache rows kc / vc
- * written for all T, att [T][n_embed].  part NULL: keys are not split. */
+ * written for all T, att [T][n_embed].  part: partials of part_floats, which
+ * limit the chunks of keys (less than a chunk's: keys are not split). */
 int lg_prefill_attn(const PfModel& M, const float* qkv, int qs, const uint16_t* kc, const uint16_t* vc, int T, int pos0,
-                    float* att, float* part, hipStream_t s);
+                    float* att, float* part, size_t part_floats, hipStream_t s);
 
 /* The layers of T prompt tokens at positions pos0.. (T <= B.tmax, tokens in
  * B.toks): KV rows pos0..pos0+T-1 written, B.x = the residual stream after

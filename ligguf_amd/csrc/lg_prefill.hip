@@ -2171,7 +2171,7 @@ int lg_prefill_layers(const PfModel& M, PfBuffers& B, int T, int pos0, hipStream
         hipLaunchKernelGGL(k_pf_qk_rope_kv, dim3((waves + 3) / 4, T), dim3(256), 0, s, B.qkv, qs, ne, kvd, L.q_norm,
                            L.k_norm, M.n_heads, M.n_kv, M.head_dim, M.rope_dim, pos0, M.rope_freq, M.eps, kc, vc);
         if ((rc = lg_check_launch("prefill qk-norm/rope/kv"))) return rc;
-        if ((rc = lg_prefill_attn(M, B.qkv, qs, kc, vc, T, pos0, B.att, B.attp, s))) return rc;
+        if ((rc = lg_prefill_attn(M, B.qkv, qs, kc, vc, T, pos0, B.att, B.ug, B.ug_floats, s))) return rc;
         if ((rc = quant(fam(L.ao), B.att, nullptr, ne, 4 * l + 1))) return rc;
         if ((rc = gemm(L.ao, ne, B.x, ne, 1))) return rc;
         /* FFN branch */

@@ -12,19 +12,50 @@ pytestmark = pytest.mark.gpu
 
 # heads, KV heads, head width (1 to 8 query heads per KV head)
 SHAPES = [(6, 6, 48), (3, 3, 128), (4, 2, 64), (12, 4, 64), (8, 2, 128), (10, 2, 64), (12, 2, 128), (14, 2, 48), (8, 1, 128)]
-# tokens, positions before: one block and its ends, an own key in the next tile, chunks that a block's first tokens
-# do not reach, a pass with keys in chunks of a few tiles
-PROMPTS = [(1, 0), (31, 0), (33, 5), (64, 64), (65, 100), (160, 450), (5, 1300), (40, 1011)]
+# tokens, positions before: one block and its ends, an own key in the next tile, keys in chunks of a few tiles; with
+# (300, 250) chunks of 384 keys of which blocks of queries see the first alone, both, and some of their tokens the second
+PROMPTS = [(1, 0), (31, 0), (33, 5), (64, 64), (65, 100), (160, 450), (5, 1300), (40, 1011), (300, 250)]
+# the same in more than 20 chunks
+LONG = [(1, 5999), (3, 6000), (40, 6037)]
 
 
 @pytest.mark.parametrize("nh,nkv,hd", SHAPES, ids=[f"{a}on{b}x{c}" for a, b, c in SHAPES])
 def test_prompt_against_steps(gpu, nh, nkv, hd):
-    ne, kvd, ctx = nh * hd, nkv * hd, 1408
+    against_steps(nh, nkv, hd, 1408, PROMPTS)
+
+
+@pytest.mark.parametrize("nh,nkv,hd", [(6, 6, 48), (8, 1, 128)], ids=["6on6x48", "8on1x128"])
+def test_many_chunks_against_steps(gpu, nh, nkv, hd):
+    against_steps(nh, nkv, hd, 6144, LONG)
+
+
+def test_first_prompt_allocates_no_partials(gpu):
+    """The partials of split keys go where up|gate's output comes later: the
+    first prompt of an engine takes the buffers of the layer pass and nothing
+    the size of the partials (17 MB here) beside them."""
+    import torch
+    ne, kvd, nff = 1024, 128, 4352
+    used = []
+    for _ in range(2):      # the first engine also loads the kernels
+        eng = Engine(0)
+        eng.load(HostModel.synthetic(ModelConfig("pfmem", 0, 1, ne, 16, 2, 64, nff, 64, 1024, 1e4, 1e-5, F32, F32, F32)))
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        eng.set_prefill_path(PREFILL_BATCHED)
+        eng.prefill(np.arange(20, dtype=np.int32), 0)
+        used.append(free - torch.cuda.mem_get_info()[0])
+        eng.close()
+    # x, qkv, attention output, up|gate and the widest activation of 512 tokens, 2 MiB steps
+    assert used[1] <= 512 * 4 * (ne + (ne + 2 * kvd) + ne + 2 * nff + nff) + 5 * 2 ** 21, used
+
+
+def against_steps(nh, nkv, hd, ctx, prompts):
+    ne, kvd = nh * hd, nkv * hd
     eng = Engine(0)
     eng.load(HostModel.synthetic(ModelConfig("pfattn", 0, 2, ne, nh, nkv, hd, 256, 64, ctx, 1e4, 1e-5, F32, F32, F32)))
     rng = np.random.default_rng(nh + hd)
     past = rng.standard_normal((2, 2, ctx, kvd)).astype(np.float16).view(np.uint16)
-    for T, pos in PROMPTS:
+    for T, pos in prompts:
         toks = rng.integers(0, 64, T).astype(np.int32)
         out = []
         for path in (PREFILL_BATCHED, PREFILL_STEPS):
