@@ -831,7 +831,7 @@ struct lg_bert {
     int8_t* aq = nullptr;
     float* ad = nullptr;
     int ldd = 0;
-    _Float16 *hx = nullptr, *hw = nullptr;   /* F16 matrices: split x / x1 and split ctx / h */
+    _Float16 *hx = nullptr, *hw = nullptr;   /* with F16 matrices: split x / x1 and split ctx / h */
     float* hinv = nullptr;                   /* [tmax] */
     /* per-pass tables: tokpos [tmax] int2, attention blocks, sequences */
     void* meta_dev = nullptr;
@@ -996,6 +996,14 @@ static int bput_mat(lg_bert* b, const lg_weight* const* ws, int n, BMat& out)
     return LG_OK;
 }
 
+/* any of the layer's Q, K and V of that type */
+static bool any_of(const BLayer& L, int type)
+{
+    for (int i = 0; i < L.nqkv; i++)
+        if (L.qkv[i].type == type) return true;
+    return false;
+}
+
 /* bound of |y_i| of a LayerNorm's output: |z_i| <= sqrt(n) */
 static float ln_bound(const float* w, const float* b, int n)
 {
@@ -1135,7 +1143,10 @@ static int bert_load_impl(lg_bert* b, const lg_bert_desc* m, int max_tokens)
             return rc;
     }
 
-    if ((rc = bert_split_scales(b, m))) return rc;
+    bool f16 = false;   /* any F16 layer matrix: split activations and their scales */
+    for (const BLayer& L : b->layers)
+        f16 = f16 || any_of(L, LG_F16) || L.ao.type == LG_F16 || L.up.type == LG_F16 || L.down.type == LG_F16;
+    if (f16 && (rc = bert_split_scales(b, m))) return rc;
 
     /* activations for tmax tokens */
     int tmax = max_tokens > 0 ? max_tokens : std::max(m->n_context, 4096);
@@ -1148,10 +1159,11 @@ static int bert_load_impl(lg_bert* b, const lg_bert_desc* m, int max_tokens)
         (rc = balloc(b, (void**)&b->y, T * ne * 4)) || (rc = balloc(b, (void**)&b->qkv, T * 3 * ne * 4)) ||
         (rc = balloc(b, (void**)&b->ctx, T * ne * 4)) || (rc = balloc(b, (void**)&b->h, T * nff * 4)) ||
         (rc = balloc(b, (void**)&b->aq, T * wmax)) || (rc = balloc(b, (void**)&b->ad, T * (wmax / 32) * 4)) ||
-        (rc = balloc(b, (void**)&b->hx, lg_hsplit_bytes((int)T, ne))) ||
-        (rc = balloc(b, (void**)&b->hw, lg_hsplit_bytes((int)T, (int)wmax))) ||
-        (rc = balloc(b, (void**)&b->hinv, T * 4)) ||
         (rc = balloc(b, (void**)&b->emb_dev, (T / 2) * ne * 4)) || (rc = balloc(b, (void**)&b->q_emb_dev, (size_t)ne * 4)))
+        return rc;
+    if (f16 && ((rc = balloc(b, (void**)&b->hx, lg_hsplit_bytes((int)T, ne))) ||
+                (rc = balloc(b, (void**)&b->hw, lg_hsplit_bytes((int)T, (int)wmax))) ||
+                (rc = balloc(b, (void**)&b->hinv, T * 4))))
         return rc;
     /* tables: tokpos T int2, attention blocks (<= T/4 + T/2) x 4 ints, sequences T/2 int2 */
     b->meta_bytes = T * 8 + (T / 4 + T / 2 + 1) * sizeof(BAttnBlk) + (T / 2) * 8;
@@ -1275,12 +1287,6 @@ static int trace_copy(const lg_bert* b, int l, int s, int K, int T)
     return LG_OK;
 }
 
-static bool any_of(const BLayer& L, int type)
-{
-    for (int i = 0; i < L.nqkv; i++)
-        if (L.qkv[i].type == type) return true;
-    return false;
-}
 static bool any_i8(const BLayer& L) { return any_of(L, BF_I8); }
 
 /* the split that a producer writes for F16 consumers (h NULL: none) */

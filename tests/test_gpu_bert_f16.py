@@ -8,8 +8,8 @@ import numpy as np
 import pytest
 
 from ligguf_amd import encode
-from ligguf_amd.bert import BERT_TINY, Bert, HostBert
-from ligguf_amd.lib import F16, F32
+from ligguf_amd.bert import BERT_TINY, Bert, BertConfig, HostBert
+from ligguf_amd.lib import F16, F32, Q8_0
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +58,22 @@ def test_split_follows_the_producer(gpu, oracle, f32):
     for s in texts(hb.cfg, [2, 40]):
         assert rel(dev.embed(s), oracle.bert_embed(hb, s)) < REL
     dev.close()
+
+
+def test_split_buffers_for_f16_only(gpu):
+    """Encoders without an F16 layer matrix have no split activations to hold:
+    4096 tokens of 384 and of 1536 values take 31 MB of them."""
+    import torch
+    cfg = BertConfig("bert-mem", 1, 384, 12, 1536, 512, 128)
+    used, devs = {}, []
+    for t in (F16, Q8_0, F16, Q8_0):      # (the first two also load the kernels)
+        hb = HostBert.synthetic(cfg.with_(layer_type=t))
+        dev = Bert(0)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        dev.load(hb, 4096)
+        used[t] = free - torch.cuda.mem_get_info()[0]
+        devs.append(dev)
+    for dev in devs:
+        dev.close()
+    assert used[Q8_0] + 24 * 2 ** 20 <= used[F16], used
