@@ -605,24 +605,27 @@ __global__ __launch_bounds__(256) void k_bert_l2norm(float* __restrict__ emb, in
 /* ------------------------------------------------------------------ */
 /* out = max over the rows (float bits) of a bound of |W_r . y + bias_r| for
  * any LayerNorm output y = z lw + lb (|z|_2 <= sqrt(K)): sqrt(K) |W_r lw|_2 +
- * sum |W_r lb| + |bias_r|.  One wave per row; *out starts at 0; a row that is
- * not finite makes it infinite. */
+ * sum |W_r lb| + |bias_r|; where the squares fall out of fp32's range, with the
+ * sum of the |W_r lw| instead of their norm.  One wave per row; *out starts at
+ * 0; a row that is not finite makes it infinite. */
 __global__ __launch_bounds__(256) void k_bert_bound(const uint16_t* __restrict__ W, int rows, int K,
                                                     const float* __restrict__ lw, const float* __restrict__ lb,
                                                     const float* __restrict__ bias, uint32_t* __restrict__ out)
 {
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= rows) return;
-    float s2 = 0.0f, s1 = 0.0f;
+    float s2 = 0.0f, s1 = 0.0f, sb = 0.0f;
     for (int i = lane; i < K; i += 64) {
         const float w = lg_h2f(W[(size_t)r * K + i]);
         s2 = __builtin_fmaf(w * lw[i], w * lw[i], s2);
-        s1 += fabsf(w * lb[i]);
+        s1 += fabsf(w * lw[i]);
+        sb += fabsf(w * lb[i]);
     }
     s2 = lg_group_sum<64>(s2);
     s1 = lg_group_sum<64>(s1);
+    sb = lg_group_sum<64>(sb);
     /* the sums' own rounding, and that of LayerNorm, is far inside the factor */
-    const float b = 1.001f * (sqrtf((float)K * s2) + s1 + fabsf(bias[r]));
+    const float b = 1.001f * (sqrtf((float)K) * (s2 > 1e-30f && s2 < INFINITY ? sqrtf(s2) : s1) + sb + fabsf(bias[r]));
     if (lane == 0) atomicMax(out, b < INFINITY ? __float_as_uint(b) : 0x7f800000u);
 }
 

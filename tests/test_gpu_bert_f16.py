@@ -41,6 +41,13 @@ def test_attention_edges(gpu, oracle, hd):
     assert np.array_equal(many.view(np.uint32), np.tile(one, (3, 1)).view(np.uint32))
 
 
+def scale(hb, norm, m, channel=slice(None)):
+    for part in ("weight", "bias"):
+        v = hb.vectors[f"{norm}.{part}"].copy()
+        v[channel] *= np.float32(m)
+        hb.vectors[f"{norm}.{part}"] = v
+
+
 @pytest.mark.parametrize("f32", [("attn_q", "attn_k", "attn_v", "ffn_up"), ("attn_v",), ("attn_output", "ffn_down"), ("ffn_up",)])
 def test_split_follows_the_producer(gpu, oracle, f32):
     cfg = BERT_TINY.with_(layer_type=F16, embd_type=F16)
@@ -49,13 +56,38 @@ def test_split_follows_the_producer(gpu, oracle, f32):
         if name.split(".")[-2] in f32:
             hb.weights[name] = (F32, rows, cols, encode.random_tensor(F32, 3, zlib.crc32(name.encode()), rows, cols, cfg.sigma))
     # LayerNorm outputs, and so the bounds, of very different sizes
-    for l, m in enumerate((1e-6, 1e4, 1.0, 30.0)):
-        for n in ("attn_output_norm.weight", "attn_output_norm.bias"):
-            if l < cfg.n_layers:
-                hb.vectors[f"blk.{l}.{n}"] = hb.vectors[f"blk.{l}.{n}"] * np.float32(m)
+    assert cfg.n_layers == 2
+    for n, m in (("token_embd_norm", 1e-3), ("blk.0.attn_output_norm", 1e-6), ("blk.0.layer_output_norm", 1e3),
+                 ("blk.1.attn_output_norm", 1e4)):
+        scale(hb, n, m)
     dev = Bert(0)
     dev.load(hb)
     for s in texts(hb.cfg, [2, 40]):
+        assert rel(dev.embed(s), oracle.bert_embed(hb, s)) < REL
+    dev.close()
+
+
+def no_bound(hb):
+    """the bound of h is no use at all (1e30 and more)"""
+    for l in range(hb.cfg.n_layers):
+        hb.vectors[f"blk.{l}.ffn_up.bias"][7] = -1e30
+
+
+def squares_underflow(hb):
+    """x1 near 1e-22: the squares in the bound of h would be zero, and h far above such a bound"""
+    scale(hb, "blk.0.attn_output_norm", 1e-22)
+    hb.vectors["blk.0.attn_output_norm.bias"][:] = 0
+    hb.vectors["blk.0.ffn_up.bias"][:] = 0
+
+
+@pytest.mark.parametrize("change", [no_bound, squares_underflow], ids=["no-bound", "squares-underflow"])
+def test_bounds_that_say_too_little(gpu, oracle, change):
+    hb = HostBert.synthetic(BERT_TINY.with_(layer_type=F16, embd_type=F16))
+    hb.vectors = {n: v.copy() for n, v in hb.vectors.items()}
+    change(hb)
+    dev = Bert(0)
+    dev.load(hb)
+    for s in texts(hb.cfg, [2, 40, 200]):
         assert rel(dev.embed(s), oracle.bert_embed(hb, s)) < REL
     dev.close()
 
