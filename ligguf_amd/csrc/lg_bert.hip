@@ -603,14 +603,13 @@ __global__ __launch_bounds__(256) void k_bert_l2norm(float* __restrict__ emb, in
 /* ------------------------------------------------------------------ */
 /* bounds of what an F16 matrix gives on LayerNorm output               */
 /* ------------------------------------------------------------------ */
-/* out = max over the rows (float bits) of a bound of |W_r . y + bias_r| for
- * any LayerNorm output y = z lw + lb (|z|_2 <= sqrt(K)): sqrt(K) |W_r lw|_2 +
- * sum |W_r lb| + |bias_r|; where the squares fall out of fp32's range, with the
- * sum of the |W_r lw| instead of their norm.  One wave per row; *out starts at
- * 0; a row that is not finite makes it infinite. */
+/* out[r] = a bound of |W_r . y + bias_r| for any LayerNorm output y = z lw +
+ * lb (|z|_2 <= sqrt(K)): sqrt(K) |W_r lw|_2 + sum |W_r lb| + |bias_r|; where
+ * the squares fall out of fp32's range, with the sum of the |W_r lw| instead
+ * of their norm.  One wave per row; not finite where something in it is not. */
 __global__ __launch_bounds__(256) void k_bert_bound(const uint16_t* __restrict__ W, int rows, int K,
                                                     const float* __restrict__ lw, const float* __restrict__ lb,
-                                                    const float* __restrict__ bias, uint32_t* __restrict__ out)
+                                                    const float* __restrict__ bias, float* __restrict__ out)
 {
     const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (r >= rows) return;
@@ -625,8 +624,8 @@ __global__ __launch_bounds__(256) void k_bert_bound(const uint16_t* __restrict__
     s1 = lg_group_sum<64>(s1);
     sb = lg_group_sum<64>(sb);
     /* the sums' own rounding, and that of LayerNorm, is far inside the factor */
-    const float b = 1.001f * (sqrtf((float)K) * (s2 > 1e-30f && s2 < INFINITY ? sqrtf(s2) : s1) + sb + fabsf(bias[r]));
-    if (lane == 0) atomicMax(out, b < INFINITY ? __float_as_uint(b) : 0x7f800000u);
+    if (lane == 0)
+        out[r] = 1.001f * (sqrtf((float)K) * (s2 > 1e-30f && s2 < INFINITY ? sqrtf(s2) : s1) + sb + fabsf(bias[r]));
 }
 
 /* ------------------------------------------------------------------ */
@@ -1007,36 +1006,45 @@ static bool any_of(const BLayer& L, int type)
     return false;
 }
 
-/* bound of |y_i| of a LayerNorm's output: |z_i| <= sqrt(n) */
-static float ln_bound(const float* w, const float* b, int n)
+/* bounds of |y_i| of a LayerNorm's output: |z_i| <= sqrt(n) */
+static std::vector<float> ln_bounds(const float* w, const float* b, int n)
 {
-    float m = 0.0f;
-    for (int i = 0; i < n; i++) {
-        const float v = sqrtf((float)n) * fabsf(w[i]) + fabsf(b[i]);
-        m = v > m || v != v ? v : m;
-        if (m != m) return INFINITY;
-    }
-    return 1.001f * m;
+    std::vector<float> v(n);
+    for (int i = 0; i < n; i++) v[i] = 1.001f * (sqrtf((float)n) * fabsf(w[i]) + fabsf(b[i]));
+    return v;
 }
 
-/* 2^-k of a split whose values stay within bound; 0: no use as one */
-static float bound_inv(float bound) { return bound < 1e30f ? lg_pow2(-lg_split_exp(bound)) : 0.0f; }
+/* 2^-k of a split whose values stay within their bounds; 0: none that serves.
+ * A split holds values to 2^-39 of its bound.  A typical value lies some
+ * sqrt(n) below its own bound: with the largest bound up to 2^10 above the
+ * median one it keeps 22 bits or, at sqrt(n) = 2^6, loses one; where one
+ * channel's bound stands out further (a neuron that a large negative bias
+ * keeps silent), each token's own maximum is taken (k_hsplit). */
+static float bounds_inv(std::vector<float> v)
+{
+    float top = 0.0f;
+    for (float x : v) {
+        if (!(x < 1e30f)) return 0.0f;
+        top = std::max(top, x);
+    }
+    v.erase(std::remove(v.begin(), v.end(), 0.0f), v.end());
+    if (v.empty()) return lg_pow2(-lg_split_exp(0.0f));
+    std::nth_element(v.begin(), v.begin() + v.size() / 2, v.end());
+    return top <= 1024.0f * v[v.size() / 2] ? lg_pow2(-lg_split_exp(top)) : 0.0f;
+}
 
 /* The scales of the split inputs of F16 matrices.  What feeds them is
  * LayerNorm output, attention -- an average of V rows -- or GELU of an F16
  * product of LayerNorm output: all bounded by the weights, so their producers
  * write the split at once instead of a pass that looks for each token's
- * largest value (k_hsplit).  A bound some 2^8 above the values a token shows
- * leaves their parts 2^-31 of them apart. */
+ * largest value (k_hsplit), unless a bound says too little (bounds_inv). */
 static int bert_split_scales(lg_bert* b, const lg_bert_desc* m)
 {
-    const int ne = b->ne;
-    uint32_t* dev = nullptr;
+    const int ne = b->ne, nff = b->nff, per = ne + nff;   /* bounds of a layer: V's rows, up's rows */
+    float* dev = nullptr;
     int rc;
-    if ((rc = balloc(b, (void**)&dev, 8 * (size_t)b->n_layers))) return rc;
-    std::vector<uint32_t> hb(2 * (size_t)b->n_layers, 0u);
-    if (b->n_layers) LG_HIP_CHECK(hipMemcpy(dev, hb.data(), hb.size() * 4, hipMemcpyHostToDevice));
-    auto bound = [&](const BMat& W, int row0, const float* lw, const float* lb, const float* bias, uint32_t* out) {
+    if ((rc = balloc(b, (void**)&dev, 4 * (size_t)per * b->n_layers))) return rc;
+    auto bound = [&](const BMat& W, int row0, const float* lw, const float* lb, const float* bias, float* out) {
         const int rows = W.rows - row0;
         hipLaunchKernelGGL(k_bert_bound, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, b->stream,
                            (const uint16_t*)W.w + (size_t)row0 * W.cols, rows, W.cols, lw, lb, bias, out);
@@ -1046,20 +1054,21 @@ static int bert_split_scales(lg_bert* b, const lg_bert_desc* m)
         const float* lw = l ? b->layers[l - 1].ln2_w : b->emb_w;
         const float* lb = l ? b->layers[l - 1].ln2_b : b->emb_b;
         const BMat& v = L.qkv[L.nqkv - 1];
-        if (v.type == LG_F16) bound(v, L.nqkv == 1 ? 2 * ne : 0, lw, lb, L.qkv_bias + 2 * ne, dev + 2 * l);
-        if (L.up.type == LG_F16) bound(L.up, 0, L.ln1_w, L.ln1_b, L.up_bias, dev + 2 * l + 1);
+        if (v.type == LG_F16) bound(v, L.nqkv == 1 ? 2 * ne : 0, lw, lb, L.qkv_bias + 2 * ne, dev + (size_t)per * l);
+        if (L.up.type == LG_F16) bound(L.up, 0, L.ln1_w, L.ln1_b, L.up_bias, dev + (size_t)per * l + ne);
     }
     if ((rc = lg_check_launch("bert bounds"))) return rc;
     LG_HIP_CHECK(hipStreamSynchronize(b->stream));
-    if (b->n_layers) LG_HIP_CHECK(hipMemcpy(hb.data(), dev, hb.size() * 4, hipMemcpyDeviceToHost));
+    std::vector<float> hb((size_t)per * b->n_layers);
+    LG_HIP_CHECK(hipMemcpy(hb.data(), dev, hb.size() * 4, hipMemcpyDeviceToHost));
     for (int l = 0; l < b->n_layers; l++) {
         BLayer& L = b->layers[l];
-        L.in_inv = bound_inv(l ? ln_bound(m->layers[l - 1].ffn_norm_w, m->layers[l - 1].ffn_norm_b, ne)
-                               : ln_bound(m->emb_norm_w, m->emb_norm_b, ne));
-        L.x1_inv = bound_inv(ln_bound(m->layers[l].attn_norm_w, m->layers[l].attn_norm_b, ne));
-        const uint32_t* u = hb.data() + 2 * l;
-        if (L.qkv[L.nqkv - 1].type == LG_F16) L.ctx_inv = bound_inv(__builtin_bit_cast(float, u[0]));
-        if (L.up.type == LG_F16) L.h_inv = bound_inv(__builtin_bit_cast(float, u[1]));
+        L.in_inv = bounds_inv(l ? ln_bounds(m->layers[l - 1].ffn_norm_w, m->layers[l - 1].ffn_norm_b, ne)
+                                : ln_bounds(m->emb_norm_w, m->emb_norm_b, ne));
+        L.x1_inv = bounds_inv(ln_bounds(m->layers[l].attn_norm_w, m->layers[l].attn_norm_b, ne));
+        const float* u = hb.data() + (size_t)per * l;
+        if (L.qkv[L.nqkv - 1].type == LG_F16) L.ctx_inv = bounds_inv({u, u + ne});
+        if (L.up.type == LG_F16) L.h_inv = bounds_inv({u + ne, u + per});
     }
     return LG_OK;
 }

@@ -67,6 +67,17 @@ def test_split_follows_the_producer(gpu, oracle, f32):
     dev.close()
 
 
+def large_norm_weight(norm):
+    """one channel of a LayerNorm far above the rest: x's or x1's split takes each token's own maximum"""
+    return lambda hb: scale(hb, norm, 2.0 ** 11, 5)
+
+
+def silent_neuron(hb):
+    """up's bias keeps one neuron at gelu = 0 and puts its bound at 1e9: the other neurons' values stay exact"""
+    for l in range(hb.cfg.n_layers):
+        hb.vectors[f"blk.{l}.ffn_up.bias"][7] = -1e9
+
+
 def no_bound(hb):
     """the bound of h is no use at all (1e30 and more)"""
     for l in range(hb.cfg.n_layers):
@@ -80,7 +91,9 @@ def squares_underflow(hb):
     hb.vectors["blk.0.ffn_up.bias"][:] = 0
 
 
-@pytest.mark.parametrize("change", [no_bound, squares_underflow], ids=["no-bound", "squares-underflow"])
+@pytest.mark.parametrize("change", [large_norm_weight("token_embd_norm"), large_norm_weight("blk.0.attn_output_norm"),
+                                    large_norm_weight("blk.0.layer_output_norm"), silent_neuron, no_bound, squares_underflow],
+                         ids=["x-of-0", "x1", "x-of-1", "silent-neuron", "no-bound", "squares-underflow"])
 def test_bounds_that_say_too_little(gpu, oracle, change):
     hb = HostBert.synthetic(BERT_TINY.with_(layer_type=F16, embd_type=F16))
     hb.vectors = {n: v.copy() for n, v in hb.vectors.items()}
