@@ -267,7 +267,7 @@ static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
     const int nrb = ((a.R + 32 * MR * WR - 1) / (32 * MR * WR) + 7) & ~7, nt = (a.T + 32 * MT * WT - 1) / (32 * MT * WT);
     const dim3 grid((unsigned)(nrb * nt)), blk(64 * WR * WT * WK);
 #define HG(E) hipLaunchKernelGGL((k_hgemm<MR, MT, WR, WT, WK, E>), grid, blk, 0, s, a, x)
-    if constexpr (WK != 2) {
+    if constexpr (MR == MT && WK != 2) {   /* the encoder's tiles (lg_hgemm) */
         switch (ep) {
         case EP_BIAS: HG(EP_BIAS); return;
         case EP_BIAS_RES: HG(EP_BIAS_RES); return;
@@ -297,7 +297,9 @@ static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
  * tokens 9.0 / 64 x 64 16.8; 1152 x 384, 260 tokens 7.7 / 7.8, 512 tokens
  * 9.5 / 8.0), 64 x 64 above (4096 tokens: 1152 x 384 24.3, 384 x 384 15.6,
  * 1536 x 384 25.9, 384 x 1536 35.4; 128 x 128 25.0, 30.7, 30.0, 50.2), and
- * 128 x 128 once it gives every CU two. */
+ * 128 x 128 once it gives every CU two: two layers of 1024 / 4096, 4096 and
+ * 8192 tokens 1006 and 1635 us (64 x 64 throughout 1143 and 2157), of 768 /
+ * 3072 755 and 1380 (804 and 1471). */
 int lg_hgemm(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
 {
     auto wgs = [&](int tr, int tt) { return (long)((a.R + tr - 1) / tr) * ((a.T + tt - 1) / tt); };

@@ -48,6 +48,25 @@ def scale(hb, norm, m, channel=slice(None)):
         hb.vectors[f"{norm}.{part}"] = v
 
 
+def test_wide_encoder_alone_and_in_a_batch(gpu, oracle):
+    """4096 tokens of 768 and 3072 values: Q|K|V and up on 128 x 128 tiles, where
+    a text alone takes 32 x 32 and 64 x 64."""
+    cfg = BERT_TINY.with_(name="bert-wide", n_layers=1, n_embed=768, n_heads=12, n_ff=3072, n_context=256, layer_type=F16,
+                          embd_type=F16)
+    hb = HostBert.synthetic(cfg)
+    dev = Bert(0)
+    dev.load(hb, 4224)
+    seqs = texts(hb.cfg, [126, 3, 200, 61] + [126] * 28 + [120])      # 4104 tokens: an uneven end
+    many = dev.embed_batch(seqs)
+    for i in (0, 1, 2, 3, 32):
+        one = dev.embed(seqs[i])
+        assert np.array_equal(one.view(np.uint32), many[i].view(np.uint32)), i
+        if i < 3:
+            ref = oracle.bert_embed(hb, seqs[i])
+            assert rel(one, ref) < REL, (i, rel(one, ref))
+    dev.close()
+
+
 @pytest.mark.parametrize("f32", [("attn_q", "attn_k", "attn_v", "ffn_up"), ("attn_v",), ("attn_output", "ffn_down"), ("ffn_up",)])
 def test_split_follows_the_producer(gpu, oracle, f32):
     cfg = BERT_TINY.with_(layer_type=F16, embd_type=F16)
