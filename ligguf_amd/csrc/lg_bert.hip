@@ -124,7 +124,7 @@ __device__ __forceinline__ void b_layernorm(float (&v)[NP][4], int n, const floa
                               : 0.0f;
         if (i0 < n) *(float4*)(out + i0) = make_float4(o[0], o[1], o[2], o[3]);
         if (q) b_emit_q8(o, q, qd, ldd, t, 4 * p + wv, n);
-        if (sp.h && i0 < n) lg_split_store4(o, 1.0f / sp.inv_all, sp, n, t, i0);
+        if (sp.h && i0 < n) lg_split_store4(o, lg_recip_pow2(sp.inv_all), sp, n, t, i0);
     }
 }
 
@@ -544,7 +544,7 @@ __global__ __launch_bounds__(256) void k_bert_attn(const float* __restrict__ qkv
     for (int i = 0; i < 4 * NDT; i += 4) {
         if (so.h) {
             const float v[4] = {r[i], r[i + 1], r[i + 2], r[i + 3]};
-            lg_split_store4(v, 1.0f / so.inv_all, so, ne, t, i0 + i);
+            lg_split_store4(v, lg_recip_pow2(so.inv_all), so, ne, t, i0 + i);
         } else {
             *(float4*)(ctx + (size_t)t * ne + i0 + i) = make_float4(r[i], r[i + 1], r[i + 2], r[i + 3]);
         }

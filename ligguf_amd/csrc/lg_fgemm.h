@@ -57,6 +57,12 @@ __host__ __device__ __forceinline__ int lg_split_exp(float amax)
 
 __host__ __device__ __forceinline__ float lg_pow2(int k) { return __builtin_bit_cast(float, (uint32_t)(127 + k) << 23); }
 
+/* 1 / x of a power of two whose reciprocal is normal too */
+__host__ __device__ __forceinline__ float lg_recip_pow2(float x)
+{
+    return __builtin_bit_cast(float, 0x7f000000u - __builtin_bit_cast(uint32_t, x));
+}
+
 /* ---- device side of the split, for the kernels that produce activations ---- */
 
 /* |x| for the maximum: infinities and NaN take no part */

@@ -58,7 +58,7 @@ __device__ __forceinline__ void hg_emit(const BGemm& a, float acc, float inv, fl
     if constexpr (EP == EP_BIAS_GELU_SPLIT) {
         /* a lane and its neighbour hold two rows of a token: the even one
          * stores both high parts, the odd one both low ones */
-        const uint32_t w = lg_split1(lg_gelu(o + bias), 1.0f / a.so.inv_all);
+        const uint32_t w = lg_split1(lg_gelu(o + bias), lg_recip_pow2(a.so.inv_all));
         const uint32_t n = (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0xb1, 0xf, 0xf, true);   /* lane ^ 1 */
         const int odd = row & 1;
         uint32_t* p = (uint32_t*)(a.so.h + (size_t)(row >> 5) * 64 + (row & 30) + 32 * odd);
@@ -78,7 +78,11 @@ __device__ __forceinline__ void hg_emit(const BGemm& a, float acc, float inv, fl
  * of MR x MT tiles of 32 x 32 (v_mfma_f32_32x32x16_f16, A = tokens, B =
  * weight rows: lane l holds token / row l % 32, values 8 (l / 32) .. +7 of a
  * 16-value step), and WK groups of such waves take consecutive parts of K
- * with stages of their own, summed in group order through LDS at the end.
+ * with stages of their own, summed in group order through LDS at the end,
+ * where each group finishes its share of the tile.  With one group doing that
+ * alone, and loads past a short part waited for, the 32 x 32 tile took 2 to 3
+ * us longer (128 x 512 with GELU, 120 tokens: 7.7 -> 4.5; the fp32 MFMA, which
+ * small models ran on before, 4.2).
  *
  * Per step of 32 values both operands go through LDS, double-buffered, a
  * step's loads in flight while the two steps before compute (one step ahead
@@ -99,10 +103,9 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
     constexpr int WB = TR * 64, XB = TT * 128, SB = WB + XB;   /* bytes of a stage */
     constexpr int NW = TR * 4 / NG, NX = TT * 8 / NG;          /* pieces per thread */
     static_assert(NW * NG == TR * 4 && NX * NG == TT * 8, "whole pieces");
-    static_assert((WK - 1) * TR * TT * 4 <= WK * 2 * SB || WK == 1, "the groups' sums fit the stages");
     __shared__ __attribute__((aligned(16))) uint8_t s_st[WK][2][SB];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int kg = wave / (WR * WT), wr = wave % (WR * WT) / WT, wt = wave % WT, gt = threadIdx.x % NG;
+    const int kg = WK == 1 ? wave / (WR * WT) : __builtin_amdgcn_readfirstlane(wave / (WR * WT)), wr = wave % (WR * WT) / WT, wt = wave % WT, gt = threadIdx.x % NG;
     const int h = lane >> 5, j = lane & 31;
     const int nt = (a.T + TT - 1) / TT;
     /* the token tiles of a row block on one XCD, 8 indices apart: its
@@ -202,7 +205,8 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
     load(s1, 1);
     store(s0, 0);
     __syncthreads();
-    for (int i = 0; i < nsg; i += 2) {
+    int i = 0;
+    for (; i < (WK == 4 ? nsg - 3 : nsg); i += 2) {
         load(s0, i + 2);
         if (PO) part(i);
         if (i < kn) compute(0);
@@ -214,49 +218,67 @@ __global__ __launch_bounds__(64 * WR * WT * WK) __attribute__((amdgpu_waves_per_
         store(s0, 0);
         __syncthreads();
     }
+    if constexpr (WK == 4) {
+        /* the last one to three steps: where a group has only a handful, no load
+         * past the last is waited for */
+        if (i + 2 < nsg) load(s0, i + 2);
+        if (i < kn) compute(0);
+        if (i + 1 < nsg) {
+            store(s1, 1);
+            __syncthreads();
+            if (i + 1 < kn) compute(1);
+            if (i + 2 < nsg) {
+                store(s0, 0);
+                __syncthreads();
+                if (i + 2 < kn) compute(0);
+            }
+        }
+        __syncthreads();
+    }
     if constexpr (PO) {
 #pragma unroll
         for (int i = 0; i < MR; i++)
 #pragma unroll
             for (int u = 0; u < MT; u++) acc[i][u] = tot[i][u] + acc[i][u];
     }
+    /* Each group ends up with 1 / WK of the tile's registers: it gives the others
+     * theirs through LDS (all stages are consumed), adds its own groups' in
+     * order, and finishes those -- the epilogue's work on all waves, not on
+     * one group's */
+    constexpr int NR = MR * MT * 16, NP = NR / WK;
+    static_assert(NR % WK == 0, "a part each");
+    float* const red = (float*)s_st;   /* [group][register][thread] */
     if constexpr (WK > 1) {
-        /* the other groups' sums, in order (all stages are consumed) */
-        float* red = (float*)s_st;
-        constexpr int NR = MR * MT * 16;
-        if (kg) {
+        static_assert(WK * NR * NG * 4 <= (int)sizeof(s_st), "the groups' sums fit the stages");
 #pragma unroll
-            for (int i = 0; i < MR; i++)
-#pragma unroll
-                for (int u = 0; u < MT; u++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) red[((kg - 1) * NR + (i * MT + u) * 16 + r) * NG + gt] = acc[i][u][r];
-        }
+        for (int f = 0; f < NR; f++)
+            if (f / NP != kg) red[(kg * NR + f) * NG + gt] = acc[f / 16 / MT][f / 16 % MT][f % 16];
         __syncthreads();
-        if (kg) return;
-#pragma unroll
-        for (int g = 0; g < WK - 1; g++)
-#pragma unroll
-            for (int i = 0; i < MR; i++)
-#pragma unroll
-                for (int u = 0; u < MT; u++)
-#pragma unroll
-                    for (int r = 0; r < 16; r++) acc[i][u][r] += red[(g * NR + (i * MT + u) * 16 + r) * NG + gt];
     }
-
 #pragma unroll
-    for (int u = 0; u < MT; u++) {
-        const int tb = t0 + (wt * MT + u) * 32 + 4 * h;   /* register r: token tb + 8 (r / 4) + r % 4 */
-        float inv[16];
+    for (int c = 0; c < WK; c++) {
+        if (WK > 1 && c != kg) continue;   /* (wave-uniform; the registers are named at compile time) */
 #pragma unroll
-        for (int r = 0; r < 16; r++) inv[r] = x.inv ? x.inv[min(tb + 8 * (r >> 2) + (r & 3), a.T - 1)] : x.inv_all;
+        for (int u = 0; u < MT; u++) {
+            const int tb = t0 + (wt * MT + u) * 32 + 4 * h;   /* register r: token tb + 8 (r / 4) + r % 4 */
+            float inv[16];
 #pragma unroll
-        for (int i = 0; i < MR; i++) {
-            const int row = r0 + (wr * MR + i) * 32 + j;
-            if (row >= a.R) continue;
-            const float bias = EP <= EP_BIAS_GELU_SPLIT ? a.bias[row] : 0.0f;
+            for (int r = 0; r < 16; r++) inv[r] = x.inv ? x.inv[min(tb + 8 * (r >> 2) + (r & 3), a.T - 1)] : x.inv_all;
 #pragma unroll
-            for (int r = 0; r < 16; r++) hg_emit<EP>(a, acc[i][u][r], inv[r], bias, tb + 8 * (r >> 2) + (r & 3), row);
+            for (int i = 0; i < MR; i++) {
+                const int row = r0 + (wr * MR + i) * 32 + j;
+                if (row >= a.R) continue;
+                const float bias = EP <= EP_BIAS_GELU_SPLIT ? a.bias[row] : 0.0f;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int f = (i * MT + u) * 16 + r;
+                    if (f / NP != c) continue;
+                    float o = c == 0 ? acc[i][u][r] : red[f * NG + gt];
+#pragma unroll
+                    for (int g = 1; g < WK; g++) o += c == g ? acc[i][u][r] : red[(g * NR + f) * NG + gt];
+                    hg_emit<EP>(a, o, inv[r], bias, tb + 8 * (r >> 2) + (r & 3), row);
+                }
+            }
         }
     }
 }
@@ -288,14 +310,14 @@ static void hgemm_launch(const BGemm& a, const HSplit& x, int ep, hipStream_t s)
  * parts where a CU would hold one workgroup only (4096 x 4096, 500 tokens 50
  * / 54 unsplit), then 64 x 64 (384 x 1536, 4096 tokens 32 / 35; split:
  * 4096 x 4096, 150 tokens 32 / 34), and 32 x 32 with K in four parts for the
- * smallest (384 x 1536, 512 tokens 8.4 / 13) and for up to 32 tokens, where
- * the weights' stream is the bound (24576 x 4096, 13 tokens 50, 4.1 TB/s;
+ * smallest (384 x 1536, 512 tokens 7.7 / 13) and for up to 32 tokens, where
+ * the weights' stream is the bound (24576 x 4096, 13 tokens 48, 4.2 TB/s;
  * 64 x 64 60).
  *
  * The encoder's matrices are narrow, and every tile must add K's four parts
  * in one order (PO above): 32 x 32 up to 384 such tiles (384 x 1536, 25
- * tokens 9.0 / 64 x 64 16.8; 1152 x 384, 260 tokens 7.7 / 7.8, 512 tokens
- * 9.5 / 8.0), 64 x 64 above (4096 tokens: 1152 x 384 24.3, 384 x 384 15.6,
+ * tokens 7.5 / 64 x 64 16.1, 1000 tokens 14.0 / 16.6; 1152 x 384, 260 tokens
+ * 5.3 / 7.1), 64 x 64 above (1536 x 384, 1000 tokens 11.1 / 9.6; 4096 tokens: 1152 x 384 24.3, 384 x 384 15.6,
  * 1536 x 384 25.9, 384 x 1536 35.4; 128 x 128 25.0, 30.7, 30.0, 50.2), and
  * 128 x 128 once it gives every CU two: two layers of 1024 / 4096, 4096 and
  * 8192 tokens 1006 and 1635 us (64 x 64 throughout 1143 and 2157), of 768 /

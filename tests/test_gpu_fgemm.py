@@ -27,8 +27,8 @@ def bound(w, x, K):
 
 
 # 32 x 32 tile and its ends; 64 x 64 with K split and unsplit; 128 x 64 split and unsplit; 128 x 128; K of one step,
-# an odd number of steps, fewer steps than K parts
-@pytest.mark.parametrize("R,K,T", [(1, 32, 1), (33, 96, 31), (32, 2016, 32), (24576, 32, 13), (100, 64, 33), (65, 12288, 64),
+# an odd number of steps, fewer steps than K parts; two to five steps a part, the last part short
+@pytest.mark.parametrize("R,K,T", [(40, 224, 20), (70, 352, 9), (33, 512, 31), (50, 608, 17), (1, 32, 1), (33, 96, 31), (32, 2016, 32), (24576, 32, 13), (100, 64, 33), (65, 12288, 64),
                                    (4095, 1056, 129), (8200, 96, 130), (6145, 416, 257), (4100, 4096, 449), (12289, 160, 193),
                                    (8193, 1024, 512)])
 def test_f16_product_tiles(gpu, R, K, T):
