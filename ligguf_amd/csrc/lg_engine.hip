@@ -1576,6 +1576,21 @@ extern "C" int lg_prefill_path(const lg_ctx* ctx)
     return ctx->pf_ok && ctx->prefill_path != LG_PREFILL_STEPS ? LG_PREFILL_BATCHED : LG_PREFILL_STEPS;
 }
 
+/* Tokens of an F16 product that are split and multiplied at a time: halves
+ * where that keeps the workspace within 2 MiB -- hipMalloc leaves its chunks
+ * beyond and takes some 27 us more -- up to 4096 columns and 10^10 products
+ * (us of a call, whole / in halves: 256 x 2048, 300 tokens 64 / 46; 1024 x
+ * 1024, 512 tokens 65 / 40; 4096 x 4096, 150 tokens 85 / 87; past the line
+ * 24576 x 2048, 300 tokens 155 / 163, 256 x 12288, 48 tokens 96 / 114; three
+ * parts 520 x 4096, 256 tokens 72 / 81; a stream-ordered allocation instead
+ * 64 -> 75, 65 -> 73). */
+static int f16_tokens_at_once(int rows, int cols, int T)
+{
+    const size_t token = lg_hsplit_bytes(1, cols) + 4, fit = (size_t)2 << 20;
+    const int half = (T + 1) / 2;
+    return token * T > fit && token * half <= fit && cols <= 4096 && (double)rows * cols * T <= 1e10 ? half : T;
+}
+
 extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, int d, const float* x, int T, float* out,
                                 void* stream)
 {
@@ -1604,12 +1619,13 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
     }
     /* workspace: quants, then scales for n/32 blocks (enough for either
      * form), the Q8_K bsums and the Q8_0 sums */
-    const int tld = (T + 3) / 4 * 4, nb = n / 256, nb0 = n / 32;
+    const int tc = at == LG_F16 ? f16_tokens_at_once(d, n, T) : T;
+    const int tld = (tc + 3) / 4 * 4, nb = n / 256, nb0 = n / 32;
     PfQ8K q = {};
     q.tld = tld;
     const size_t o_d = (size_t)tld * n, o_bs = o_d + (size_t)nb0 * tld * 4, o_as = o_bs + (size_t)tld * nb * 32;
-    const size_t o_inv = lg_hsplit_bytes(T, n);   /* F16 form: the two parts, then a scale per token */
-    const size_t bytes = at == LG_F16 ? o_inv + (size_t)T * 4 : o_as + (size_t)nb0 * tld * 4;
+    const size_t o_inv = lg_hsplit_bytes(tc, n);   /* F16 form: the two parts, then a scale per token */
+    const size_t bytes = at == LG_F16 ? o_inv + (size_t)tc * 4 : o_as + (size_t)nb0 * tld * 4;
     uint8_t* ws = nullptr;
     const hipError_t e = hipMalloc((void**)&ws, bytes);
     if (e != hipSuccess) { lg_set_error("matmul_tokens: hipMalloc(%zu): %s", bytes, hipGetErrorString(e)); return LG_ERR_NOMEM; }
@@ -1618,8 +1634,12 @@ extern "C" int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, in
     q.bs = (int16_t*)(ws + o_bs);
     q.as = (int*)(ws + o_as);
     if (at == LG_F16) q.hs = HSplit{(_Float16*)ws, (float*)(ws + o_inv), 0.0f};
-    int rc = lg_prefill_quantize(at, x, n, nullptr, 0.0f, n, T, q, (hipStream_t)stream);
-    if (!rc) rc = lg_prefill_gemm(type, (const uint8_t*)w, rsz, d, n, q, T, out, d, 0, (hipStream_t)stream);
+    int rc = LG_OK;
+    for (int t = 0; !rc && t < T; t += tc) {   /* (the workspace's next use follows on the stream) */
+        const int m = std::min(tc, T - t);
+        rc = lg_prefill_quantize(at, x + (size_t)t * n, n, nullptr, 0.0f, n, m, q, (hipStream_t)stream);
+        if (!rc) rc = lg_prefill_gemm(type, (const uint8_t*)w, rsz, d, n, q, m, out + (size_t)t * d, d, 0, (hipStream_t)stream);
+    }
     const hipError_t e2 = hipStreamSynchronize((hipStream_t)stream);
     (void)hipFree(ws);
     if (!rc && e2 != hipSuccess) { lg_set_error("matmul_tokens: %s", hipGetErrorString(e2)); rc = LG_ERR_HIP; }

@@ -26,11 +26,14 @@ def bound(w, x, K):
     return (2.0 ** -21 + 6 * (K / 16 + 4) ** 0.5 * 2.0 ** -24) * terms + 2.0 ** -38 * peak
 
 
-# 32 x 32 tile and its ends; 64 x 64 with K split and unsplit; 128 x 64 split and unsplit; 128 x 128; K of one step,
-# an odd number of steps, fewer steps than K parts; two to five steps a part, the last part short
-@pytest.mark.parametrize("R,K,T", [(40, 224, 20), (70, 352, 9), (33, 512, 31), (50, 608, 17), (1, 32, 1), (33, 96, 31), (32, 2016, 32), (24576, 32, 13), (100, 64, 33), (65, 12288, 64),
+# 32 x 32 tile and its ends, a part of K of one to five steps, fewer steps than parts, the last part short, few rows
+# and many; 64 x 64 with K split and unsplit; 128 x 64 split and unsplit; 128 x 128; either side of where
+# the tokens are taken in halves, uneven ones
+@pytest.mark.parametrize("R,K,T", [(100001, 96, 31), (40003, 224, 32), (26001, 352, 31), (18001, 512, 32), (15001, 608, 32),
+                                   (40, 224, 20), (70, 352, 9), (33, 512, 31), (50, 608, 17),
+                                   (1, 32, 1), (33, 96, 31), (32, 2016, 32), (24576, 32, 13), (100, 64, 33), (65, 12288, 64),
                                    (4095, 1056, 129), (8200, 96, 130), (6145, 416, 257), (4100, 4096, 449), (12289, 160, 193),
-                                   (8193, 1024, 512)])
+                                   (8193, 1024, 512), (1024, 1024, 511), (1024, 1024, 512), (520, 4096, 127), (520, 4096, 150)])
 def test_f16_product_tiles(gpu, R, K, T):
     g = torch.Generator(device="cuda").manual_seed(R + K + T)
     w = (torch.randn(R, K, generator=g, device=gpu) * 0.02).half()
