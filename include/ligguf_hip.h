@@ -249,8 +249,8 @@ int lg_prefill(lg_ctx* ctx, const int* toks, int n, int pos0, float* logits_host
  * layer type -- Q2_K..Q6_K, Q8_0, Q1_0, Q1_G on int8 MFMA, F16 on fp16
  * MFMA (each fp32 activation as two fp16 parts), F32 on fp32 MFMA, in any
  * mix (a Q4_K_M-style model with Q6_K matrices among its Q4_K ones included)
- * -- and needs head_dim 48, 64 or 128 with 1, 2, 4 or 8 query heads per KV
- * head.  STEPS: one decode step per token, bit-equal to n lg_decode_step calls.  AUTO (the
+ * -- and needs head_dim 48, 64 or 128 with 1 to 8 query heads per KV head.
+ * STEPS: one decode step per token, bit-equal to n lg_decode_step calls.  AUTO (the
  * default): BATCHED when the model allows it and n >= 2, else STEPS.
  * lg_prefill_path reports what a prompt of 2+ tokens takes (-1 without a
  * model). */
@@ -306,15 +306,16 @@ int lg_quantize_q8_K(const float* x, int64_t n, void* y, void* stream);
 int lg_matvec(int type, const void* w, uint32_t rsz, int n, int d, const void* xq, float* out, int accumulate,
               void* stream);
 
-/* The matvec of T tokens at once on int8 MFMA (the batched prefill's GEMMs):
- * out[t*d + r] = row r of w . Q(x[t*n ..]) for t < T, r < d, each fp32 row
+/* The matvec of T tokens at once (the batched prefill's GEMMs: int8 MFMA for
+ * quantized weights): out[t*d + r] = row r of w . Q(x[t*n ..]) for t < T, r < d, each fp32 row
  * of x quantized as quantize_q8_K (K-quant weights, n % 256 == 0) or
  * quantize_q8_0 (Q8_0, Q1_0, Q1_G weights; n % 32 == 0, n % 256 for Q1_G)
  * does, or taken as fp32 (F32 weights on fp32 MFMA, F16 weights on fp16 MFMA
  * with each value in two fp16 parts; n % 32 == 0).  The
  * integer block sums are those of lg_matvec (the dot products of
  * fast/lil_math.cpp:397-739); only the fp32 accumulation order differs.  Allocates and frees a workspace of
- * about 1.3*T*n bytes and synchronizes `stream` (tests and benches).  No
+ * about 1.4*T*n bytes (F16: 4*T*n, or half of that for half the tokens at a
+ * time; F32: none) and synchronizes `stream` (tests and benches).  No
  * counterpart in the reference, which calls matmul per token. */
 int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, int d, const float* x, int T, float* out,
                      void* stream);

@@ -1562,7 +1562,7 @@ extern "C" int lg_set_prefill_path(lg_ctx* ctx, int path)
         return ctx_fail(ctx, LG_ERR_ARG);
     }
     if (path == LG_PREFILL_BATCHED && ctx->loaded && !ctx->pf_ok) {
-        lg_set_error("set_prefill_path: the batched prefill needs head_dim 48, 64 or 128 with 1, 2, 4 or 8 query "
+        lg_set_error("set_prefill_path: the batched prefill needs head_dim 48, 64 or 128 with 1 to 8 query "
                      "heads per KV head");
         return ctx_fail(ctx, LG_ERR_TYPE);
     }

@@ -21,10 +21,10 @@ struct HSplit {
 };
 
 struct BGemm {
-    const uint8_t* w;          /* F32/F16: [R][K]; BF_I8: int8 [R][K] */
+    const uint8_t* w;          /* F16 (lg_hgemm), F32: [R][K]; BF_I8: int8 [R][K] */
     const float* wd;           /* BF_I8: [K/32][R] */
     int R, K;
-    const float* x;            /* fp32 activations [T][ldx] (F32/F16) */
+    const float* x;            /* fp32 activations [T][ldx] (F32) */
     int ldx;
     const int8_t* q;           /* Q8_0 activations [T][K] (BF_I8) */
     const float* qd;           /* [K/32][ldd] */

@@ -49,7 +49,7 @@ typedef _Float16 v8h __attribute__((ext_vector_type(8)));
  * bytes per product, wrote V^T two bytes at a time and never split the keys
  * (32 heads of 128, 8 KV heads): 512 tokens after 6900..7412, 352 us -> 147
  * (410 TFLOP/s of the products asked for, 820 issued with the split parts);
- * 512 after none 30 -> 23 and 5.6 to merge.  All 64 scores of a column in one
+ * 512 after none 30 -> 21 and 5.6 to merge.  All 64 scores of a column in one
  * softmax step rather than 32 and 32: 157 -> 147 us there.
  *
  * Long contexts split the keys over workgroups as well (nsplit chunks of ck
@@ -411,8 +411,9 @@ __global__ __launch_bounds__(256) void k_pf_attn_merge(const float* __restrict__
  * would start when the first ends), each of at least PF_ATT_KEYS keys, below
  * which a chunk's start and the merge cost what they save: two 4096-wide
  * layers, 3 tokens after 6000, 367 us with 1024 keys a chunk, 342 with 512,
- * 329 with 256, 332 with 128; 512 tokens after none 833 with 512, 829 with
- * 256. */
+ * 329 with 256, 332 with 128.  Two chunks begin to pay near 512 keys: a
+ * prompt of 512 after none 813 us in one or two, of 64 after 450 367 / 361,
+ * 300 after 600 680 / 666 (in three). */
 constexpr int PF_ATT_WGS = 256, PF_ATT_KEYS = 256;
 static int pf_attn_split(int T, int keys, int n_kv)
 {

@@ -198,9 +198,8 @@ def test_bert_minilm_shape(dev, oracle):
 
 
 def test_bert_long_sequences(dev, oracle):
-    """the attention variants by sequence length: up to 512 and up to 1024
-    positions on MFMA with the score rows in LDS, longer ones on the
-    vector-ALU kernel with fewer queries per block; a batch mixing them"""
+    """long sequences, whose key steps the four waves of a workgroup share, at
+    lengths up to the context; a batch mixing them"""
     hb = load(dev, HostBert.synthetic(BERT_TINY.with_(n_context=2048, seed=21)))
     rng = np.random.default_rng(12)
     seqs = [rng.integers(5, hb.cfg.vocab, n) for n in (300, 700, 1500, 2046)]

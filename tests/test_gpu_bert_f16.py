@@ -2,6 +2,7 @@
 16-query blocks and 32-key steps, every head width, a wave or a workgroup to
 a query block, alone and in a batch bit for bit (other tiles of the products), and activations split by their producer (bounds of the weights)
 or from each token's own maximum (F32 producers, bounds that are none)."""
+import gc
 import zlib
 
 import numpy as np
@@ -133,6 +134,7 @@ def test_split_buffers_for_f16_only(gpu):
     for t in (F16, Q8_0, F16, Q8_0):      # (the first two also load the kernels)
         hb = HostBert.synthetic(cfg.with_(layer_type=t))
         dev = Bert(0)
+        gc.collect()      # what earlier tests left goes back now, not in between
         torch.cuda.synchronize()
         free = torch.cuda.mem_get_info()[0]
         dev.load(hb, 4096)

@@ -2,6 +2,8 @@
 64- or 32-key tiles, with keys in one and in several chunks, for every number
 of query heads per KV head and head width: a prompt in one pass against the
 token-sequential path, over an unquantized model of two layers."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -39,6 +41,7 @@ def test_first_prompt_allocates_no_partials(gpu):
     for _ in range(2):      # the first engine also loads the kernels
         eng = Engine(0)
         eng.load(HostModel.synthetic(ModelConfig("pfmem", 0, 1, ne, 16, 2, 64, nff, 64, 1024, 1e4, 1e-5, F32, F32, F32)))
+        gc.collect()      # what earlier tests left goes back now, not in between
         torch.cuda.synchronize()
         free = torch.cuda.mem_get_info()[0]
         eng.set_prefill_path(PREFILL_BATCHED)

@@ -72,8 +72,8 @@ GEMM_CASES = [(t, d, n, T) for t in (Q2_K, Q3_K, Q5_K, Q6_K)
 def test_matmul_tokens_types_vs_oracle(gpu, oracle, wt, d, n, T):
     """The K-quant GEMM (one int8 MFMA per 16- or 32-value sub-block, the
     sub-block scales in int32), the Q8_0 / Q1_0 GEMM (one per 32-value
-    block, widths any multiple of 32) and the F16 / F32 GEMM (fp32 MFMA on
-    the unquantized activation) against the oracle's matvec of each token."""
+    block, widths any multiple of 32), the F16 GEMM (fp16 MFMA, each fp32
+    activation in two parts) and the F32 one (fp32 MFMA) against the oracle's matvec of each token."""
     rng = np.random.default_rng(d + n + T + wt)
     w = encode.random_tensor(wt, d + n + wt, wt, d, n)
     x = rng.standard_normal((T, n)).astype(np.float32)
