@@ -320,9 +320,9 @@ int lg_matvec(int type, const void* w, uint32_t rsz, int n, int d, const void* x
 int lg_matmul_tokens(int type, const void* w, uint32_t rsz, int n, int d, const float* x, int T, float* out,
                      void* stream);
 /* the tile that the int8 GEMMs of lg_prefill and lg_matmul_tokens take for a
- * rows x cols matrix times T tokens: weight rows and tokens of a workgroup,
- * parts of K (tests; needs no GPU) */
-int lg_prefill_tile(int rows, int cols, int T, int* tile_rows, int* tile_tokens, int* k_parts);
+ * rows x cols matrix of a quantized type times T tokens: weight rows and
+ * tokens of a workgroup, parts of K (tests; needs no GPU) */
+int lg_prefill_tile(int type, int rows, int cols, int T, int* tile_rows, int* tile_tokens, int* k_parts);
 
 /* rmsnorm (fast/lil_math.cpp:922-929) fused with the activation quantizer
  * that follows it in inference() (:37-39): out_q gets Q8_K (qtype LG_Q8_K),

@@ -971,38 +971,47 @@ bool lg_prefill_gemm16() { return pf_gemm16(); }
  * that has nothing to compute still walks its steps, so
  *   cost = p start + steps parts (p / 2 pair + p % 2 alone)
  * gives the tile: smaller workgroups fill more CUs and walk less of K each,
- * larger ones unpack a weight for more tokens and write each sum once.  The
- * table (units of about 0.07 us for Q4_K, 0.25 for Q8_0) is one least
- * regret over 12 row forms, 96 to 24576 rows, 256 to 12544 columns and 2 to
- * 512 tokens, each tile timed with weights from HBM (3013 shapes): the tile
- * taken is 0.4 % above the fastest in the mean, and none is slower than 128 x
- * 64 with K in two parts up to 256 workgroups and from 1024 columns, the
- * choice before these tiles, which is 35 % above the fastest.  us at the
- * tile taken / at that choice:
- *    4096 x 4096, 257..448 tokens  Q4_K 27..33 (both; 64 x 32 in two 31..43), Q5_K 37..42 (both; 42..58)
+ * larger ones unpack a weight for more tokens and write each sum once.  Two
+ * tables: one for the K-quants and for the 34- and 6-byte blocks of GGUF rows,
+ * one for the other 32-value rows, whose 16-byte loads are aligned and cost
+ * as much alone as in pairs (units of some 0.03 us for Q4_K, 0.13 for Q8_0).
+ * Each is the one of least regret over 12 row forms, 96 to 24576 rows, 256 to
+ * 12544 columns and 2 to 512 tokens, every tile timed with weights from HBM
+ * and with the same weights again (6484 shapes): the tile taken is 0.4 %
+ * above the fastest in the mean.  128 x 64 with K in two parts up to 256
+ * workgroups and from 1024 columns, the one choice there was, is 65 % above
+ * it, and faster than the tile taken by more than 2 % at 4 of them (1.03).
+ * us at the tile taken / at that choice, weights from HBM:
+ *    4096 x 4096, 257..417 tokens  Q4_K 27..33 (both; 64 x 32 in two 31..43), Q5_K 37..42 (both; 42..58)
  *    4096 x 12288, 77 tokens       Q4_K 35 / 72, Q6_K 59 / 117, Q8_0 96 / 206
- *    6144 x 4096, 77 tokens        Q4_K 21 / 25, Q1_G 30 / 47
+ *    6144 x 4096, 77 tokens        Q4_K 20 / 25, Q1_G 30 / 47
  *    4096 x 12288, 16 tokens       Q4_K 23 / 64, Q6_K 36 / 111, Q1_G 36 / 130
  *    4096 x 512, 200 tokens        Q6_K 9.4 (128 x 64 unsplit; 64 x 32 in two 11.9) */
 struct PfTile {
-    int rows, tokens, parts, start, alone, pair;
+    int rows, tokens, parts;
+};
+struct PfCost {
+    int start, alone, pair;
 };
 enum { PF_T128x64, PF_T128x64_K2, PF_T64x32_K2, PF_T64x32_K4, PF_T32x32_K4, PF_TILES };
-static constexpr PfTile pf_tiles[PF_TILES] = {
-    {128, 64, 1, 24, 20, 30}, {128, 64, 2, 32, 16, 35}, {64, 32, 2, 20, 8, 13}, {64, 32, 4, 30, 6, 13}, {32, 32, 4, 18, 5, 7}};
+static constexpr PfTile pf_tiles[PF_TILES] = {{128, 64, 1}, {128, 64, 2}, {64, 32, 2}, {64, 32, 4}, {32, 32, 4}};
+static constexpr PfCost pf_cost[2][PF_TILES] = {{{38, 44, 63}, {62, 35, 80}, {37, 15, 26}, {74, 12, 26}, {35, 8, 16}},
+                                                {{39, 53, 53}, {68, 39, 82}, {28, 15, 23}, {43, 12, 27}, {32, 9, 13}}};
 
-static int pf_tile(int rows, int cols, int T)
+static int pf_tile(int wtype, int rows, int cols, int T)
 {
+    const PfCost* cost = pf_cost[wtype == LG_Q1_G || wtype == LG_Q1_G_R || wtype == LG_Q1_0_R || wtype == LG_Q8_0_R];
     int best = 0;
     long low = 0;
     for (int i = 0; i < PF_TILES; i++) {
         const PfTile& t = pf_tiles[i];
+        const PfCost& c = cost[i];
         /* the launch pads the row blocks to a multiple of 8 (the XCDs) */
         const long wgs = (long)(((rows + t.rows - 1) / t.rows + 7) & ~7) * ((T + t.tokens - 1) / t.tokens);
         const long p = (wgs + 255) / 256, steps = ((cols + 255) / 256 + t.parts - 1) / t.parts;
-        const long cost = p * t.start + steps * t.parts * (p / 2 * t.pair + p % 2 * t.alone);
-        if (i == 0 || cost < low) {
-            low = cost;
+        const long sum = p * c.start + steps * t.parts * (p / 2 * c.pair + p % 2 * c.alone);
+        if (i == 0 || sum < low) {
+            low = sum;
             best = i;
         }
     }
@@ -1010,13 +1019,14 @@ static int pf_tile(int rows, int cols, int T)
 }
 
 /* (tests) the tile the int8 GEMMs take for rows x cols times T tokens */
-extern "C" int lg_prefill_tile(int rows, int cols, int T, int* tile_rows, int* tile_tokens, int* k_parts)
+extern "C" int lg_prefill_tile(int wtype, int rows, int cols, int T, int* tile_rows, int* tile_tokens, int* k_parts)
 {
-    if (rows <= 0 || cols <= 0 || T <= 0 || !tile_rows || !tile_tokens || !k_parts) {
+    const int at = lg_prefill_act_type(wtype);
+    if ((at != LG_Q8_K && at != LG_Q8_0) || rows <= 0 || cols <= 0 || T <= 0 || !tile_rows || !tile_tokens || !k_parts) {
         lg_set_error("prefill tile: bad arguments");
         return LG_ERR_ARG;
     }
-    const PfTile& t = pf_tiles[pf_tile(rows, cols, T)];
+    const PfTile& t = pf_tiles[pf_tile(wtype, rows, cols, T)];
     *tile_rows = t.rows;
     *tile_tokens = t.tokens;
     *k_parts = t.parts;
@@ -1038,7 +1048,7 @@ static int gemm_k32(const uint8_t* W, uint32_t rsz, int rows, int cols, const Pf
                     int accumulate, hipStream_t s)
 {
 #define K32(RW, KS, TT) k32_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
-    switch (pf_tile(rows, cols, T)) {
+    switch (pf_tile(WT, rows, cols, T)) {
     case PF_T128x64: K32(4, 1, 64); break;
     case PF_T128x64_K2: K32(4, 2, 64); break;
     case PF_T64x32_K2: K32(2, 2, 32); break;
@@ -1973,7 +1983,7 @@ static int gemm_b32x(const uint8_t* W, uint32_t rsz, int rows, int cols, const P
                      int accumulate, hipStream_t s)
 {
 #define B32X(RW, KS, TT) b32x_launch<WT, RW, KS, TT>(W, rsz, rows, cols, x, T, out, ldo, accumulate, s)
-    switch (pf_tile(rows, cols, T)) {
+    switch (pf_tile(WT, rows, cols, T)) {
     case PF_T128x64: B32X(4, 1, 64); break;
     case PF_T128x64_K2: B32X(4, 2, 64); break;
     case PF_T64x32_K2: B32X(2, 2, 32); break;

@@ -100,7 +100,7 @@ SIGNATURES = {
     "lg_quantize_q8_K": (C.c_int, [_vp, C.c_int64, _vp, _vp]),
     "lg_matvec": (C.c_int, [C.c_int, _vp, C.c_uint32, C.c_int, C.c_int, _vp, _vp, C.c_int, _vp]),
     "lg_matmul_tokens": (C.c_int, [C.c_int, _vp, C.c_uint32, C.c_int, C.c_int, _vp, C.c_int, _vp, _vp]),
-    "lg_prefill_tile": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]),
+    "lg_prefill_tile": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "lg_rmsnorm_quant": (C.c_int, [_vp, _vp, C.c_int, C.c_float, C.c_int, _vp, _vp, _vp]),
     "lg_qk_norm_rope_kv": (C.c_int, [_vp, _vp, _vp, _vp, _vp, C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, _vp,
                                      C.c_float, _vp, _vp, _vp]),

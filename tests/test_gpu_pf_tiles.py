@@ -13,12 +13,13 @@ from ligguf_amd.lib import Q1_0, Q1_G, Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, TYPE_
 
 pytestmark = pytest.mark.gpu
 
-# rows, width, tokens, the tile taken (rows x tokens, parts of K): ends of rows and tokens, one step of K in two parts,
-# as many steps as parts and fewer, an uneven last part
-SHAPES = [(33, 256, 1, (64, 32, 2)), (600, 2304, 95, (32, 32, 4)), (4090, 1280, 33, (32, 32, 4)), (65, 768, 40, (32, 32, 4)),
-          (4097, 512, 65, (64, 32, 2)), (4065, 1280, 100, (64, 32, 2)), (4033, 1792, 97, (64, 32, 4)),
-          (3970, 2304, 449, (128, 64, 2)), (6145, 768, 100, (128, 64, 1)), (3970, 1280, 449, (128, 64, 1)),
-          (12289, 512, 165, (128, 64, 1))]
+# rows, width, tokens, the tile taken (rows x tokens, parts of K) and Q1_G's where it is another one: ends of rows and
+# tokens, one step of K in two parts, as many steps as parts and fewer, an uneven last part
+SHAPES = [(33, 256, 1, (64, 32, 2), None), (600, 2304, 95, (32, 32, 4), None), (4090, 1280, 33, (32, 32, 4), None),
+          (65, 768, 40, (32, 32, 4), None), (4097, 512, 65, (64, 32, 2), None), (4065, 1280, 100, (64, 32, 2), None),
+          (4033, 1792, 97, (64, 32, 2), (64, 32, 4)), (4097, 4864, 65, (64, 32, 4), None), (3970, 2304, 449, (128, 64, 2), None),
+          (6145, 768, 100, (128, 64, 1), (64, 32, 2)), (3970, 1280, 449, (128, 64, 1), (128, 64, 2)),
+          (12289, 512, 165, (128, 64, 1), None)]
 TYPES = [Q2_K, Q3_K, Q4_K, Q5_K, Q6_K, Q8_0, Q1_0, Q1_G]
 
 
@@ -34,10 +35,11 @@ def activations(x, kq):
 
 
 @pytest.mark.parametrize("wt", TYPES, ids=[TYPE_NAMES[t] for t in TYPES])
-@pytest.mark.parametrize("R,n,T,tile", SHAPES)
-def test_tiles(gpu, wt, R, n, T, tile):
+@pytest.mark.parametrize("R,n,T,tile,q1g", SHAPES)
+def test_tiles(gpu, wt, R, n, T, tile, q1g):
     got = [C.c_int() for _ in range(3)]
-    assert load().lg_prefill_tile(R, n, T, *(C.byref(o) for o in got)) == 0 and tuple(o.value for o in got) == tile
+    assert load().lg_prefill_tile(wt, R, n, T, *(C.byref(o) for o in got)) == 0
+    assert tuple(o.value for o in got) == (q1g if q1g and wt == Q1_G else tile)
     rsz = row_size(wt, n)
     distinct = min(R, 512)   # encoding is host work: the rows repeat, with a stride that no tile edge divides
     rows = encode.random_tensor(wt, R + n, wt, distinct, n).reshape(distinct, rsz)
