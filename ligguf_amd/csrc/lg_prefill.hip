@@ -984,7 +984,7 @@ bool lg_prefill_gemm16() { return pf_gemm16(); }
  * us at the tile taken / at that choice, weights from HBM:
  *    4096 x 4096, 257..417 tokens  Q4_K 27..33 (both; 64 x 32 in two 31..43), Q5_K 37..42 (both; 42..58)
  *    4096 x 12288, 77 tokens       Q4_K 35 / 72, Q6_K 59 / 117, Q8_0 96 / 206
- *    6144 x 4096, 77 tokens        Q4_K 20 / 25, Q1_G 30 / 47
+ *    6144 x 4096, 77 tokens        Q4_K 21 / 25, Q1_G 31 / 47
  *    4096 x 12288, 16 tokens       Q4_K 23 / 64, Q6_K 36 / 111, Q1_G 36 / 130
  *    4096 x 512, 200 tokens        Q6_K 9.4 (128 x 64 unsplit; 64 x 32 in two 11.9) */
 struct PfTile {
